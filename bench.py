@@ -37,19 +37,17 @@ HBM_PEAK_GBS = 8000.0
 # (ED_Q_MIXED_KERNEL; None for FP64), strip height, item order) -- the tile order changes the bytes.
 TRAFFIC_MEASURED = {
     ("C", "mixed", 3, 4, 0): (127743801.0 * 2.0 + 3239083.4) * 1024,  # contract_mixed_ws_kernel<3>, 8 timeslices
-    ("C", "fp64", None, 2, 0): (434679524.2 * 2.0 + 2751779.8) * 1024,  # contract_kernel<double, 3>, 8 timeslices
     # contract_mixed16_kernel<2> (the tuned mixed kernel), 8 timeslices:
     # profiles/elemental_32c64_nev200_tuned_kernel_trace.md
     ("C", "mixed", 5, 2, 1): (180556618.2 * 2.0 + 3430244.9) * 1024,
 }
 TRAFFIC_SOURCE = {
     ("C", "mixed", 3, 4, 0): "profiles/elemental_32c64_nev200_hbm_traffic.md",
-    ("C", "fp64", None, 2, 0): "profiles/elemental_32c64_nev200_hbm_traffic.md",
     ("C", "mixed", 5, 2, 1): "profiles/elemental_32c64_nev200_tuned_kernel_trace.md",
 }
 # the library's ED_Q_MIXED_KERNEL answer -> the kernel the mixed form runs
 MIXED_KERNEL = {
-    0: "contract_kernel<double, 3>",
+    0: "f64::contract_kernel",
     1: "contract_kernel<float, 3>",
     2: "contract_mixed_f16_kernel<3>",
     3: "contract_mixed_ws_kernel<3>",
@@ -726,7 +724,7 @@ def main():
             "frac": (r["contract_fp16_tflops"] / PEAK_FP16) if all_f16 else r["contract_tflops_executed"] / PEAK[head],
             "traffic": TRAFFIC_MEASURED.get(traffic_key),
             "traffic_source": TRAFFIC_SOURCE.get(traffic_key),
-            "kernel": MIXED_KERNEL[r["mixed_kernel"]] if head == "mixed" else "contract_kernel<double, 3>",
+            "kernel": MIXED_KERNEL[r["mixed_kernel"]] if head == "mixed" else "f64::contract_kernel",
             "flops_basis": (
                 "executed FP16 MFMA flops of the factorized contraction per launch (split sum and phase "
                 "contraction both on FP16 MFMA with hi/lo operand splits)"
@@ -734,7 +732,7 @@ def main():
                 else "executed MFMA flops of the factorized contraction per launch; the mixed kernel's FP16 "
                 "MFMA flops are converted to FP32-equivalent at the FP32:FP16 peak ratio 157.3:2500"
                 if head == "mixed"
-                else "executed FP64 MFMA flops of the factorized contraction per launch"
+                else "executed FP64 multiply-adds (matrix split sum, vector x sums) of the factorized contraction per launch"
             ),
             "executed_flops_per_launch": r["executed_flops_per_launch"],
             "avg_launch_ms": r["contract_ms_per_launch"],

@@ -3,6 +3,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <array>
 #include <cmath>
 #include <cstdarg>
 #include <cstdio>
@@ -17,6 +18,7 @@
 #include "../../include/elemental_hip.h"
 #include "ed_kernels.hpp"
 #include "ed_mixed16.hpp"
+#include "ed_fp64.hpp"
 #include "ed_gauge.hpp"
 #include "ed_adjoint.hpp"
 
@@ -173,7 +175,6 @@ struct ed_context {
   DevBuf<SplitTerm> splits_u;
   DevBuf<int> pidx;  // plus [npb*16] then minus [npb*16]
   DevBuf<double> psum;  // [npb*16] sum over sites of Phi_b
-  DevBuf<double> ph64;
   DevBuf<float> ph32;
   DevBuf<ed::half8> ph16;  // [npb][V3P/32][4][16][32] fp16 hi/lo of 2^14 Phi
   int mixed_stage2 = -1;   // 1: FP16 three-term split, 0: FP32 MFMA, -1: FP16 from V3 >= 4096 on
@@ -190,6 +191,24 @@ struct ed_context {
   int wsh = 0;             // scale exponent of the FP16 stage-1 workspace
   int W_elem = 0;          // bytes per complex element of the data now in W (0: none)
   uint64_t gen = 0;        // bumped whenever buffers or plan a captured launch refers to change
+
+  // FP64 contraction (ed_fp64.hpp): tile groups of one derivative for three
+  // strip heights, and one launch per block of momenta
+  struct MomBlock {
+    int pat = 0, nf = 0, ns = 0, nmom = 0;
+    size_t xt = 0, yt = 0, zt = 0, zslot = 0, mt = 0;  // elements into their tables in ftab
+  };
+  std::vector<MomBlock> fblocks;
+  int f_nt = 1, f_gt = 0, f_ns = 1;           // tiles per workgroup, groups per t, most product slots
+  int f_nsplit = 1, f_pps = 1, f_spp = 1, f_lps = 1;  // line ranges (ed::f64::Args)
+  int f_ngrp[3][2] = {};            // [strip variant][all tiles, te <= tf]
+  size_t f_grp0[3][2] = {};         // first group of each list
+  int64_t f_macs = 0;               // multiply-adds of one timeslice
+  DevBuf<char> ftab;                // axis functions, then MomTerm, Group and slot tables
+  size_t f_mt = 0, f_grp = 0, f_slot = 0;  // byte offsets of the last three
+  DevBuf<double> M;                 // moments of a batch
+  DevBuf<double> Mfix;              // moments of ed_compute_noalloc, allocated with the plan
+  int fix_tb = 0;                   // timeslices Mfix holds
 
   // reverse pass
   int bns_max = 1;        // largest merged split count of one derivative
@@ -336,6 +355,357 @@ std::vector<SplitTerm> merged_splits(const std::vector<int>& t) {
 void adj_shape(int ns, int& rb, int& gc) {
   rb = ns <= 1 ? 4 : ns <= 2 ? ED_ADJ_RB2 : ns <= 4 ? 2 : 1;
   gc = 8 / rb > 4 ? 4 : 8 / rb;
+}
+
+// Tile groups of one derivative over nt x nt tiles (all of them, or those with
+// te <= tf), at most four tiles and six row blocks each, in strips of hb
+// blocks of 2 x 2 tiles: consecutive groups share row blocks in an XCD's L2.
+// An odd last row or column of tiles goes in runs of four, and the three tiles
+// of a diagonal block take a fourth one from the last column or from every
+// fourth diagonal block, so that few of a workgroup's waves idle.
+std::vector<ed::f64::Group> tile_groups(int nt, bool tri, int hb) {
+  std::vector<ed::f64::Group> out;
+  typedef std::vector<std::pair<int, int>> Tiles;
+  auto add = [&](const Tiles& t) {
+    ed::f64::Group g{};
+    for (auto& p : t) {
+      int l = 0, r = 0;
+      while (l < g.nL && g.rowL[l] != p.first) ++l;
+      if (l == g.nL) g.rowL[g.nL++] = (short)p.first;
+      while (r < g.nR && g.rowR[r] != p.second) ++r;
+      if (r == g.nR) g.rowR[g.nR++] = (short)p.second;
+      g.tile[g.nT++] = (short)(l | r << 4);
+    }
+    out.push_back(g);
+  };
+  if (nt == 1) {
+    add({{0, 0}});
+    return out;
+  }
+  const int m = nt / 2, last = nt - 1;
+  const bool odd = nt & 1;
+  for (int s = 0; s < m; s += hb)
+    for (int bf = tri ? s : 0; bf < m; ++bf)
+      for (int be = s; be < std::min(s + hb, m); ++be) {
+        const int e = 2 * be, f = 2 * bf;
+        if (!tri || be < bf) add({{e, f}, {e, f + 1}, {e + 1, f}, {e + 1, f + 1}});
+      }
+  auto runs = [&](const Tiles& t) {
+    for (size_t k = 0; k < t.size(); k += 4) add(Tiles(t.begin() + k, t.begin() + std::min(t.size(), k + 4)));
+  };
+  Tiles col, row;
+  if (tri) {
+    auto diag = [](int b) { return Tiles{{2 * b, 2 * b}, {2 * b, 2 * b + 1}, {2 * b + 1, 2 * b + 1}}; };
+    for (int b = 0; b < m; ++b) {
+      Tiles t = diag(b);
+      if (odd) {
+        t.push_back({2 * b, last});
+        col.push_back({2 * b + 1, last});
+      } else if (b % 4 == 3) {
+        continue;  // its tiles went to the three blocks before it
+      } else if (b / 4 * 4 + 3 < m) {
+        t.push_back(diag(b / 4 * 4 + 3)[b % 4]);
+      }
+      add(t);
+    }
+    if (odd) col.push_back({last, last});
+    runs(col);
+  } else if (odd) {
+    for (int f = 0; f < nt; ++f) row.push_back({last, f});
+    for (int e = 0; e < last; ++e) col.push_back({e, last});
+    runs(row);
+    runs(col);
+  }
+  return out;
+}
+
+// cos and sin of 2 pi n x / L, exact at multiples of a quarter turn
+void axis_phase(long n, int x, int L, double& co, double& si) {
+  const long k = (n * x) % L;
+  if (k == 0) co = 1.0, si = 0.0;
+  else if (2 * k == L) co = -1.0, si = 0.0;
+  else if (4 * k == L) co = 0.0, si = 1.0;
+  else if (4 * k == 3L * L) co = 0.0, si = -1.0;
+  else {
+    const double a = 2.0 * M_PI * ((double)k / L);
+    co = std::cos(a);
+    si = std::sin(a);
+  }
+}
+
+const std::vector<std::vector<int>>& f64_patterns() {
+  static const std::vector<std::vector<int>> p = {{1}, {3, 1, 1}, {3, 3, 3}, {5, 3, 3, 1, 1}, {7, 5, 5}, {5, 5, 1, 1}};
+  return p;
+}
+
+// Momentum blocks, tile groups and line ranges of the FP64 contraction.
+//
+// Momenta (nx, ny, nz) that agree in |nx| and |ny| use the same products of x
+// and y functions; such a class goes into one block as a whole (its z
+// functions are split over blocks only past NF_MAX moments), so each block's
+// momenta come from its own moments.  Blocks take, of the compiled slot
+// patterns, the one that covers most moments with the fewest slots: 1, 7, 19,
+// 27 and 33 momenta of |n|^2 <= 0 ... 4 need one block, |n|^2 <= 9 two.
+void plan_fp64(ed_context* c, std::vector<DPlan>& dpl) {
+  const int P = (int)(c->moms.size() / 3);
+  typedef std::pair<int, int> Cls;
+  std::map<int, std::map<int, std::map<int, std::vector<int>>>> left;  // |nx| -> |ny| -> |nz| -> momenta
+  for (int p = 0; p < P; ++p) {
+    const int32_t* n = &c->moms[3 * p];
+    left[std::abs(n[0])][std::abs(n[1])][std::abs(n[2])].push_back(p);
+  }
+  std::vector<double> tab;
+  std::vector<int> slots;
+  std::vector<ed::f64::MomTerm> mts;
+  c->fblocks.clear();
+  c->f_ns = 1;
+  auto two = [](int n) { return n ? 2 : 1; };
+  auto value = [](int n, int sine, int x, int L) {
+    double co, si;
+    axis_phase(n, x, L, co, si);
+    return sine ? si : co;
+  };
+  while (!left.empty()) {
+    struct Trial {
+      int pat = 0, nf = 0, ns = 0;
+      std::vector<std::pair<int, int>> xf;                 // x function of each position: (|nx|, sine), -1 unused
+      std::vector<std::pair<Cls, std::vector<int>>> take;  // class -> its |nz| taken
+    } best;
+    const auto& pats = f64_patterns();
+    for (size_t ip = 0; ip < pats.size(); ++ip) {
+      const std::vector<int>& cap = pats[ip];
+      Trial t;
+      t.pat = (int)ip;
+      t.xf.assign(cap.size(), {-1, 0});
+      for (int v : cap) t.ns += v;
+      // |nx| by the number of y functions it needs, most first
+      std::vector<std::pair<int, int>> order;
+      for (auto& gx : left) {
+        int need = 0;
+        for (auto& gy : gx.second) need += two(gy.first);
+        order.push_back({-need, gx.first});
+      }
+      std::sort(order.begin(), order.end());
+      size_t pos = 0;
+      for (auto& o : order) {
+        const int nx = o.second, w = two(nx);
+        if (pos + w > cap.size()) continue;
+        int room = cap[pos + w - 1];  // capacities do not increase
+        bool any = false;
+        for (auto& gy : left[nx]) {
+          if (two(gy.first) > room) continue;
+          std::vector<int> nz;
+          for (auto& gz : gy.second) {
+            const int add = w * two(gy.first) * two(gz.first);
+            if (t.nf + add > ed::f64::NF_MAX) break;
+            t.nf += add;
+            nz.push_back(gz.first);
+          }
+          if (nz.empty()) continue;
+          room -= two(gy.first);
+          t.take.push_back({{nx, gy.first}, nz});
+          any = true;
+        }
+        if (any)
+          for (int i = 0; i < w; ++i) t.xf[pos++] = {nx, i};
+      }
+      if (t.nf > best.nf || (t.nf == best.nf && t.ns < best.ns)) best = t;
+    }
+    // tables of the block: slots of position i in the order its classes came
+    const std::vector<int>& cap = pats[best.pat];
+    ed_context::MomBlock b;
+    b.pat = best.pat;
+    b.nf = best.nf;
+    b.ns = best.ns;
+    const int F1 = (int)cap.size(), NS = best.ns;
+    std::vector<std::pair<int, int>> yf(NS, {-1, 0});     // y function of each slot
+    std::vector<std::vector<std::pair<int, int>>> zf(NS);  // z functions of each slot
+    std::map<std::array<int, 4>, int> slot_of;            // (|nx|, sine x, |ny|, sine y) -> slot
+    for (int i = 0, s0 = 0; i < F1; s0 += cap[i++]) {
+      int k = s0;
+      for (auto& tk : best.take) {
+        if (tk.first.first != best.xf[i].first) continue;
+        for (int sy = 0; sy < two(tk.first.second); ++sy, ++k) {
+          yf[k] = {tk.first.second, sy};
+          slot_of[{best.xf[i].first, best.xf[i].second, tk.first.second, sy}] = k;
+          for (int nz : tk.second)
+            for (int sz = 0; sz < two(nz); ++sz) zf[k].push_back({nz, sz});
+        }
+      }
+    }
+    b.xt = tab.size();
+    for (int x = 0; x < c->Lx; ++x)
+      for (auto& f : best.xf) tab.push_back(f.first < 0 ? 0.0 : value(f.first, f.second, x, c->Lx));
+    tab.insert(tab.end(), F1, 0.0);  // read by the second half of an odd line's last pair
+    b.yt = tab.size();
+    for (int y = 0; y < c->Ly; ++y)
+      for (auto& f : yf) tab.push_back(f.first < 0 ? 0.0 : value(f.first, f.second, y, c->Ly));
+    b.zt = tab.size();
+    for (int z = 0; z < c->Lz; ++z)
+      for (auto& zk : zf)
+        for (auto& f : zk) tab.push_back(value(f.first, f.second, z, c->Lz));
+    tab.insert(tab.end(), 8, 0.0);  // read past the last plane's moments
+    b.zslot = slots.size();
+    std::vector<int> z0(1, 0);
+    for (auto& zk : zf) z0.push_back(z0.back() + (int)zk.size());
+    slots.insert(slots.end(), z0.begin(), z0.end());
+    b.mt = mts.size();
+    for (auto& tk : best.take)
+      for (int nz : tk.second) {
+        auto& ps = left[tk.first.first][tk.first.second][nz];
+        for (int p : ps) {
+          const int32_t* n = &c->moms[3 * p];
+          ed::f64::MomTerm mt{};
+          mt.p = p;
+          for (int sx = 0; sx < two(n[0]); ++sx)
+            for (int sy = 0; sy < two(n[1]); ++sy)
+              for (int sz = 0; sz < two(n[2]); ++sz) {
+                const int k = slot_of[{std::abs(n[0]), sx, std::abs(n[1]), sy}];
+                int j = 0;
+                while (zf[k][j] != std::make_pair(std::abs(n[2]), sz)) ++j;
+                const int neg = (sx && n[0] < 0) + (sy && n[1] < 0) + (sz && n[2] < 0);
+                mt.k[mt.n] = (short)(z0[k] + j);
+                mt.code[mt.n++] = (short)((sx + sy + sz + 2 * neg) & 3);
+              }
+          mts.push_back(mt);
+        }
+        left[tk.first.first][tk.first.second].erase(nz);
+        if (left[tk.first.first][tk.first.second].empty()) left[tk.first.first].erase(tk.first.second);
+        if (left[tk.first.first].empty()) left.erase(tk.first.first);
+      }
+    b.nmom = (int)(mts.size() - b.mt);
+    c->f_ns = std::max(c->f_ns, b.ns);
+    c->fblocks.push_back(b);
+  }
+  // tile groups for strips of 1, 2 and 4 blocks
+  const int nt = c->NeP / 16;
+  c->f_nt = nt == 1 ? 1 : ed::f64::NT_MAX;
+  std::vector<ed::f64::Group> grp;
+  for (int v = 0; v < 3; ++v) {
+    for (int tri = 0; tri < 2; ++tri) {
+      const auto g = tile_groups(nt, tri != 0, 1 << v);
+      c->f_grp0[v][tri] = grp.size();
+      c->f_ngrp[v][tri] = (int)g.size();
+      grp.insert(grp.end(), g.begin(), g.end());
+    }
+  }
+  // the strip variants order the same groups, so one numbering serves all
+  c->f_gt = 0;
+  c->f_macs = 0;
+  for (DPlan& p : dpl) {
+    p.grp0 = c->f_gt;
+    c->f_gt += c->f_ngrp[0][p.mirror];
+    const int64_t tiles = p.mirror ? nt * (nt + 1) / 2 : nt * nt;
+    for (auto& b : c->fblocks)
+      c->f_macs += tiles * c->V3 * (2 * 1024 * ((6 * p.nsplit + 3) / 4) + 512 * (int64_t)f64_patterns()[b.pat].size());
+  }
+  // Line ranges.  Whole planes: 4096 workgroups over eight timeslices (or all of
+  // a shorter lattice; 16 a CU, against an uneven end of the launch), more where
+  // a range keeps 4096 sites; parts of a plane, of at least 64 sites, only where
+  // whole planes give fewer than 1024 workgroups.  Measured: 32^3, Nev 200 with
+  // 1, 2, 8 ranges 190.8, 186.9, 181.9 ms per eight timeslices; 16^3, Nev 100
+  // with 2, 8, 16 ranges 8.76, 8.12, 8.19 ms; 20^3, Nev 70 in planes and half
+  // planes 2.16 and 2.38 ms; one timeslice of 16^3, Nev 64 in planes and half
+  // planes 0.65 and 0.61 ms.  The ranges depend on the shape alone, so a
+  // timeslice gives the same bits in every batch.
+  const int64_t one = (int64_t)c->f_gt * (int64_t)c->fblocks.size() * std::min(c->Lt, 8);
+  const int64_t planes = std::max<int64_t>((4096 + one - 1) / one, c->V3 / 4096);  // plane ranges asked for
+  if (one * c->Lz >= 1024) {
+    const int n = (int)std::min<int64_t>(planes, c->Lz);
+    c->f_pps = (c->Lz + n - 1) / n;
+    c->f_spp = 1;
+  } else {
+    const int64_t parts = (1024 + one * c->Lz - 1) / (one * c->Lz);
+    const int most = std::max(1, c->Lx * c->Ly / 64);
+    c->f_pps = 1;
+    c->f_spp = (int)std::min<int64_t>({parts, (int64_t)most, (int64_t)c->Ly});
+  }
+  c->f_lps = (c->Ly + c->f_spp - 1) / c->f_spp;
+  c->f_spp = (c->Ly + c->f_lps - 1) / c->f_lps;
+  c->f_nsplit = c->f_spp > 1 ? c->Lz * c->f_spp : (c->Lz + c->f_pps - 1) / c->f_pps;
+
+  std::vector<char> buf;
+  auto put = [&](const void* p, size_t bytes) {
+    const size_t at = (buf.size() + 15) / 16 * 16;
+    buf.resize(at + bytes);
+    std::memcpy(buf.data() + at, p, bytes);
+    return at;
+  };
+  put(tab.data(), tab.size() * sizeof(double));
+  c->f_mt = put(mts.data(), mts.size() * sizeof(mts[0]));
+  c->f_grp = put(grp.data(), grp.size() * sizeof(grp[0]));
+  c->f_slot = put(slots.data(), slots.size() * sizeof(int));
+  c->ftab.ensure(buf.size());
+  HIPCHK(hipMemcpy(c->ftab.p, buf.data(), buf.size(), hipMemcpyHostToDevice));
+}
+
+// doubles of x-y sums per timeslice
+size_t moments_per_t(const ed_context* c) {
+  return (size_t)c->f_gt * c->Lz * c->f_spp * c->f_nt * 2 * c->f_ns * 256;
+}
+
+// The FP64 contraction of nb timeslices in W, into out from timeslice t_out0
+// on: per momentum block the moments, then the momenta.
+template <class L>
+void enqueue_fp64(ed_context* c, const double2* W, int nb, int t_out0, double2* out, double* M, hipStream_t st,
+                  L&& launch) {
+  const int v = c->strip <= 2 ? 0 : c->strip <= 4 ? 1 : 2;  // strip heights in blocks of two tiles
+  ed::f64::Args a{};
+  a.g = c->geom(c->slots());
+  a.D = c->D;
+  a.P = (int)(c->moms.size() / 3);
+  a.nd = c->nd;
+  a.gt = c->f_gt;
+  a.NT = c->f_nt;
+  a.nsplit = c->f_nsplit;
+  a.pps = c->f_pps;
+  a.spp = c->f_spp;
+  a.lps = c->f_lps;
+  a.nwork = nb * c->f_gt * c->f_nsplit;
+  a.order = c->item_order;
+  a.t_out0 = t_out0;
+  a.dplan = c->dplan.p;
+  a.splits = c->splits.p;
+  for (int k = 0; k < 2; ++k) {
+    a.ngrp[k] = c->f_ngrp[v][k];
+    a.grp[k] = (const ed::f64::Group*)(const void*)(c->ftab.p + c->f_grp) + c->f_grp0[v][k];
+  }
+  a.wgt = c->use_wgt ? c->wgt.p : nullptr;
+  a.M = M;
+  a.out = out;
+  if (c->nsplit_max > 8) fail(ED_ERR_UNSUPPORTED, "derivative with %d split terms", c->nsplit_max);
+  const size_t lds = ed::f64::lds_of(c->f_nt);
+  launch(ED_KERNEL_CONTRACT, [&] {
+    for (const auto& b : c->fblocks) {
+      a.nf = b.nf;
+      a.ns = b.ns;
+      a.nmom = b.nmom;
+      const double* tab = (const double*)(const void*)c->ftab.p;
+      a.xt = tab + b.xt;
+      a.yt = tab + b.yt;
+      a.zt = tab + b.zt;
+      a.zslot = (const int*)(const void*)(c->ftab.p + c->f_slot) + b.zslot;
+      a.mt = (const ed::f64::MomTerm*)(const void*)(c->ftab.p + c->f_mt) + b.mt;
+      auto go = [&](auto pat) {
+        using PAT = decltype(pat);
+        if (c->nsplit_max > 4)
+          ed::f64::contract_kernel<PAT, 12><<<a.nwork, 128 * a.NT, lds, st>>>(W, a);
+        else
+          ed::f64::contract_kernel<PAT, 6><<<a.nwork, 128 * a.NT, lds, st>>>(W, a);
+      };
+      switch (b.pat) {
+        case 0: go(ed::f64::Pattern<1>{}); break;
+        case 1: go(ed::f64::Pattern<3, 1, 1>{}); break;
+        case 2: go(ed::f64::Pattern<3, 3, 3>{}); break;
+        case 3: go(ed::f64::Pattern<5, 3, 3, 1, 1>{}); break;
+        case 4: go(ed::f64::Pattern<7, 5, 5>{}); break;
+        default: go(ed::f64::Pattern<5, 5, 1, 1>{}); break;
+      }
+      HIPCHK(hipGetLastError());
+      ed::f64::momenta_kernel<<<nb * c->f_gt * a.NT * 4, 256, (size_t)2 * b.nf * 64 * sizeof(double), st>>>(a);
+      HIPCHK(hipGetLastError());
+    }
+  });
 }
 
 void build_plan(ed_context* c) {
@@ -507,6 +877,8 @@ void build_plan(ed_context* c) {
     c->items_t = items;
   }
 
+  plan_fp64(c, dpl);
+
   // Unit plan of the FP16 stage-1 kernel.  A merged split's coefficient is
   // (-1)^{|nR|} times a positive multiplicity (merged_splits).  With slot n
   // of the workspace stored times i^{|n|} (the hop multiplies each child by
@@ -550,15 +922,12 @@ void build_plan(ed_context* c) {
   c->splits.ensure(std::max<size_t>(1, sp.size()));
   c->pidx.ensure(idx.size());
   c->psum.ensure(ps.size());
-  c->ph64.ensure(2 * pr.size());
   c->ph32.ensure(2 * pr.size());
   c->ph16.ensure(p16.size() / 8);
   HIPCHK(hipMemcpy(c->dplan.p, dpl.data(), dpl.size() * sizeof(DPlan), hipMemcpyHostToDevice));
   if (!sp.empty()) HIPCHK(hipMemcpy(c->splits.p, sp.data(), sp.size() * sizeof(SplitTerm), hipMemcpyHostToDevice));
   HIPCHK(hipMemcpy(c->pidx.p, idx.data(), idx.size() * sizeof(int), hipMemcpyHostToDevice));
   HIPCHK(hipMemcpy(c->psum.p, ps.data(), ps.size() * sizeof(double), hipMemcpyHostToDevice));
-  HIPCHK(hipMemcpy(c->ph64.p, pr.data(), pr.size() * sizeof(double), hipMemcpyHostToDevice));
-  HIPCHK(hipMemcpy(c->ph64.p + pr.size(), pi.data(), pi.size() * sizeof(double), hipMemcpyHostToDevice));
   HIPCHK(hipMemcpy(c->ph32.p, pr32.data(), pr32.size() * sizeof(float), hipMemcpyHostToDevice));
   HIPCHK(hipMemcpy(c->ph32.p + pr32.size(), pi32.data(), pi32.size() * sizeof(float), hipMemcpyHostToDevice));
   HIPCHK(hipMemcpy(c->ph16.p, p16.data(), p16.size() * sizeof(_Float16), hipMemcpyHostToDevice));
@@ -637,6 +1006,17 @@ void build_plan(ed_context* c) {
     HIPCHK(hipMemcpy(c->bgroups.p, grp.data(), grp.size() * sizeof(int2), hipMemcpyHostToDevice));
     HIPCHK(hipMemcpy(c->phase_grp.p, pa.data(), pa.size() * sizeof(double2), hipMemcpyHostToDevice));
     HIPCHK(hipMemcpy(c->child_of.p, child.data(), child.size() * sizeof(int), hipMemcpyHostToDevice));
+  }
+  // moments of ed_compute_noalloc, which cannot allocate: up to eight
+  // timeslices within 16 MiB, at least one, for lattices its workspace holds
+  c->fix_tb = 0;
+  if ((size_t)c->slots() * c->NeP * 3 * c->V3P * sizeof(double2) <= ED_NOALLOC_SCRATCH_BYTES) {
+    const size_t per_t = moments_per_t(c);
+    const size_t n = std::max<size_t>(1, std::min<size_t>({(size_t)8, (size_t)c->Lt, ((size_t)2 << 20) / per_t}));
+    c->Mfix.ensure(n * per_t);
+    c->fix_tb = (int)n;
+  } else {
+    c->Mfix.reset();
   }
   c->plan_dirty = false;
   ++c->gen;
@@ -802,9 +1182,10 @@ int auto_tbatch(const ed_context* c, int nt) {
     // of the free device memory, so a shared or crowded GPU gets smaller
     // batches instead of a failed allocation
     size_t free_b = 0, total_b = 0;
-    if (hipMemGetInfo(&free_b, &total_b) == hipSuccess) budget = std::min(budget, c->W.n + free_b / 4 * 3);
+    const size_t held = c->W.n + c->M.n * sizeof(double);
+    if (hipMemGetInfo(&free_b, &total_b) == hipSuccess) budget = std::min(budget, held + free_b / 4 * 3);
     const size_t per_t = per_t_ws_bytes<T>(c);
-    TB = (int)std::max<size_t>(1, budget / per_t);
+    TB = (int)std::max<size_t>(1, budget / (per_t + (sizeof(T) == 8 ? moments_per_t(c) * sizeof(double) : 0)));
     // whole timeslices per XCD: the contraction hands each of the 8 XCDs a
     // contiguous eighth of the work items, and the items of one timeslice
     // differ in cost by derivative.  Large timeslices (>= 1 GiB of
@@ -904,10 +1285,6 @@ __global__ void zero_fill_kernel(uint4* __restrict__ p, size_t n) {
 template <typename T>
 void run_batches(ed_context* c, int t0, int nt, double2* out_dev, void* out_host, char* fixed = nullptr,
                  size_t fixed_bytes = 0) {
-  const T* ph = nullptr;
-  if (sizeof(T) == 8) ph = (const T*)(void*)c->ph64.p;
-  else ph = (const T*)(void*)c->ph32.p;
-  const size_t phn = (size_t)c->npb * 16 * c->V3P;
   const bool noalloc = fixed != nullptr;
   int TB;
   ed::c_t<T>* W;
@@ -919,6 +1296,7 @@ void run_batches(ed_context* c, int t0, int nt, double2* out_dev, void* out_host
            "(use ed_compute)", per_t, fixed_bytes);
     TB = std::min<int>(nt, (int)std::min<size_t>(fixed_bytes / per_t, (size_t)nt));
     if (c->tbatch_opt > 0) TB = std::min(TB, c->tbatch_opt);
+    if (sizeof(T) == 8) TB = std::min(TB, c->fix_tb);
     W = (ed::c_t<T>*)(void*)fixed;
     const size_t n16 = per_t * TB / sizeof(uint4);
     zero_fill_kernel<<<(unsigned)std::min<size_t>(4096, (n16 + 255) / 256), 256, 0, c->stream>>>((uint4*)(void*)fixed,
@@ -927,6 +1305,7 @@ void run_batches(ed_context* c, int t0, int nt, double2* out_dev, void* out_host
   } else {
     TB = auto_tbatch<T>(c, nt);
     W = ensure_workspace<T>(c, TB);
+    if (sizeof(T) == 8) c->M.ensure(moments_per_t(c) * TB);
   }
   const size_t out_t = (size_t)c->D * (c->moms.size() / 3) * c->Ne * c->Ne;
 
@@ -946,9 +1325,13 @@ void run_batches(ed_context* c, int t0, int nt, double2* out_dev, void* out_host
 
   for (int tb0 = t0; tb0 < t0 + nt; tb0 += TB) {
     const int nb = std::min(TB, t0 + nt - tb0);
+    if constexpr (sizeof(T) == 8) {
+      enqueue_stencil<T>(c, W, tb0, nb, c->stream, launch);
+      enqueue_fp64(c, W, nb, out_dev ? (tb0 - t0) : 0, out, noalloc ? c->Mfix.p : c->M.p, c->stream, launch);
+    } else {
     ContractArgs a = contract_args(c, nb, out_dev ? (tb0 - t0) : 0);
     const int nblk = (a.nwork + 7) / 8 * 8;
-    if (sizeof(T) == 4 && use_h16(c)) {
+    if (use_h16(c)) {
       // the same bytes hold the hi/lo FP16 pairs; padding stays zero in both forms
       uint2* Wh = (uint2*)(void*)W;
       c->wsh = h16_shift(c);
@@ -967,7 +1350,7 @@ void run_batches(ed_context* c, int t0, int nt, double2* out_dev, void* out_host
       });
     } else {
     enqueue_stencil<T>(c, W, tb0, nb, c->stream, launch);
-    if (sizeof(T) == 4 && use_f16_stage2(c)) {
+    if (use_f16_stage2(c)) {
       const float2* Wf = (const float2*)(const void*)W;
       launch(ED_KERNEL_CONTRACT, [&] {
         if (use_ws_kernel(c)) {
@@ -998,6 +1381,8 @@ void run_batches(ed_context* c, int t0, int nt, double2* out_dev, void* out_host
       });
     } else
     launch(ED_KERNEL_CONTRACT, [&] {
+      const float* ph = c->ph32.p;
+      const size_t phn = (size_t)c->npb * 16 * c->V3P;
       if (c->nks_max <= 1)
         ed::contract_kernel<T, 1><<<nblk, 64 * ed::NWAVE, 0, c->stream>>>(W, ph, ph + phn, out, a);
       else if (c->nks_max <= 2)
@@ -1009,6 +1394,7 @@ void run_batches(ed_context* c, int t0, int nt, double2* out_dev, void* out_host
       else
         fail(ED_ERR_UNSUPPORTED, "derivative with %d split terms", 4 * c->nks_max / 3);
     });
+    }
     }
     if (!out_dev) {
       HIPCHK(hipMemcpyAsync((double2*)out_host + (size_t)(tb0 - t0) * out_t, out, (size_t)nb * out_t * sizeof(double2),
@@ -1303,6 +1689,7 @@ std::vector<uint64_t> batch_prepare(ed_batch* b) {
     build_plan(c);
     const int kind = batch_kind(b, c, it.mode);
     void* W = kind == 0 ? (void*)ensure_workspace<double>(c, c->Lt) : (void*)ensure_workspace<float>(c, c->Lt);
+    if (kind == 0) c->M.ensure(moments_per_t(c) * c->Lt);
     ed::GroupProblem gp{};
     gp.a = contract_args(c, c->Lt, 0);
     if (b->strip > 0) gp.a.strip = b->strip;
@@ -1317,11 +1704,7 @@ std::vector<uint64_t> batch_prepare(ed_batch* b) {
       }
     }
     gp.W = W;
-    if (kind == 0) {
-      const size_t phn = (size_t)c->npb * 16 * c->V3P;
-      gp.ph0 = c->ph64.p;
-      gp.ph1 = c->ph64.p + phn;
-    } else if (kind == 1) {
+    if (kind == 1) {
       const size_t phn = (size_t)c->npb * 16 * c->V3P;
       gp.ph0 = c->ph32.p;
       gp.ph1 = c->ph32.p + phn;
@@ -1331,7 +1714,7 @@ std::vector<uint64_t> batch_prepare(ed_batch* b) {
     }
     gp.out = it.out;
     gp.work0 = b->total[kind];
-    tab[kind].push_back(gp);
+    if (kind) tab[kind].push_back(gp);  // FP64 members run their own launches
     b->nks[kind] = std::max(b->nks[kind], kind == 3 ? h16_groups(c) : c->nks_max);
     if (kind == 2 && ws_wide(c)) b->wide = true;
     fp.push_back((uint64_t)(uintptr_t)c);
@@ -1340,6 +1723,8 @@ std::vector<uint64_t> batch_prepare(ed_batch* b) {
     fp.push_back((uint64_t)(uintptr_t)c->U64.p);
     fp.push_back((uint64_t)(uintptr_t)c->V.p);
     fp.push_back((uint64_t)(uintptr_t)c->V64.p);
+    fp.push_back((uint64_t)(uintptr_t)c->M.p);
+    fp.push_back((uint64_t)(uintptr_t)it.out);
     fp.push_back((uint64_t)kind);
     fp.push_back((uint64_t)(int64_t)c->wsh);
     int64_t tot = (int64_t)b->total[kind] + gp.a.nwork;
@@ -1388,9 +1773,10 @@ void batch_enqueue(ed_batch* b) {
   for (auto& it : b->items) {
     ed_context* c = it.ctx;
     const int kind = batch_kind(b, c, it.mode);
-    if (kind == 0)
+    if (kind == 0) {
       enqueue_stencil<double>(c, (double2*)(void*)c->W.p, 0, c->Lt, b->stream, direct);
-    else if (kind == 3)
+      enqueue_fp64(c, (const double2*)(void*)c->W.p, c->Lt, 0, it.out, c->M.p, b->stream, direct);
+    } else if (kind == 3)
       enqueue_stencil<ed::hsplit>(c, (uint2*)(void*)c->W.p, 0, c->Lt, b->stream, direct);
     else
       enqueue_stencil<float>(c, (float2*)(void*)c->W.p, 0, c->Lt, b->stream, direct);
@@ -1408,7 +1794,7 @@ void batch_enqueue(ed_batch* b) {
                                                                                     b->order);
     HIPCHK(hipGetLastError());
   }
-  for (int k = 0; k < 3; ++k) {
+  for (int k = 1; k < 3; ++k) {
     if (!b->nprob[k]) continue;
     const int grid = batch_grid(b, b->total[k]);
     const ed::GroupProblem* P = b->probs[k].p;
@@ -1418,8 +1804,7 @@ void batch_enqueue(ed_batch* b) {
     const bool wide = k == 2 && b->wide;  // ks <= 3 then (batch_prepare)
 #define ED_GROUP(KS, WD)                                                                                   \
   do {                                                                                                     \
-    if (k == 0) ed::contract_group_kernel<double, KS><<<grid, blk, 0, b->stream>>>(P, np, tot, ord);      \
-    else if (k == 1) ed::contract_group_kernel<float, KS><<<grid, blk, 0, b->stream>>>(P, np, tot, ord);  \
+    if (k == 1) ed::contract_group_kernel<float, KS><<<grid, blk, 0, b->stream>>>(P, np, tot, ord);  \
     else if (b->grid_per_cu <= 0) ed::contract_mixed_item_kernel<KS, WD><<<grid, blk, 0, b->stream>>>(P, np, tot, ord); \
     else ed::contract_mixed_group_kernel<KS, WD><<<grid, blk, 0, b->stream>>>(P, np, tot, ord);           \
   } while (0)
@@ -1581,6 +1966,7 @@ int ed_set_lattice(ed_context* ctx, int Lx, int Ly, int Lz, int Lt, int Ne) {
     ctx->use_wgt = false;
     ctx->plan_dirty = true;
     ctx->W.reset();
+    ctx->M.reset();
     ctx->W_elem = 0;
     ctx->stage.reset();
     ctx->bW.reset();
@@ -1719,6 +2105,7 @@ int ed_set_derivatives(ed_context* ctx, int num_nabla) {
     ctx->D = level_start(num_nabla + 1);
     ctx->plan_dirty = true;
     ctx->W.reset();
+    ctx->M.reset();
     ctx->W_elem = 0;
     ctx->stage.reset();
     ctx->bW.reset();
@@ -1737,6 +2124,7 @@ int ed_set_displacement(ed_context* ctx, int distance) {
     ctx->D = distance + 1;
     ctx->plan_dirty = true;
     ctx->W.reset();
+    ctx->M.reset();
     ctx->W_elem = 0;
     ctx->stage.reset();
     ctx->bW.reset();
@@ -1886,16 +2274,9 @@ int ed_query(ed_context* ctx, int what, int64_t* value) {
     // the upper triangle for palindromic ones
     const int64_t nt = ctx->NeP / 16, tiles[2] = {nt * nt, nt * (nt + 1) / 2};
     auto tw = [&](const int64_t (&v)[2]) { return tiles[0] * v[0] + tiles[1] * v[1]; };
-    const int64_t chunks = ctx->V3P / ed::SC;
     const int64_t P = (int64_t)(ctx->moms.size() / 3);
     switch (what) {
-      case ED_Q_CONTRACT_FLOPS_PER_T: {
-        // per work item and chunk: stage 1 (16 sites x 4 MFMAs per k-step) and
-        // stage 2 (4 waves x 4 k-steps x 4 N-blocks x 4 real products)
-        const int64_t mf = ctx->npb * chunks * (tw(ctx->mfma_per_chunk_stage1) + tw(ctx->nd_tri) * 256);
-        *value = mf * 2 * 16 * 16 * 4;
-        break;
-      }
+      case ED_Q_CONTRACT_FLOPS_PER_T: *value = 2 * ctx->f_macs; break;
       case ED_Q_MIXED_F32_FLOPS_PER_T:
       case ED_Q_MIXED_F16_FLOPS_PER_T: {
         // the mixed FP16 kernel: per (tile, d, 32-site chunk) stage 1 has 32 * 4 * nks(d)

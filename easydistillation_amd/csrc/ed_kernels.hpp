@@ -541,6 +541,7 @@ struct DPlan {
                     // writes the transposed tile (tf, te) through the partner rule
   int item0;        // first work item of this d within a timeslice
   int rot;          // the FP16 stage-1 kernel multiplies its result by i^rot
+  int grp0;         // FP64 contraction: first tile group of this d within a timeslice
 };
 
 // The diagonal tile of a self-partnered derivative computes every (e, f)
@@ -577,7 +578,7 @@ struct ContractArgs {
 // within an f-tile the strip's rows, so 32 consecutive items (one per CU of
 // an XCD, started together) read about TS e slabs and 32 / TS f slabs of the
 // workspace, which then hit in that XCD's L2 (TS = 4 for the mixed kernels,
-// 2 for the FP64/FP32 kernel, measured, and the defaults; ContractArgs::strip
+// 2 for the FP32 kernel, measured, and the defaults; ContractArgs::strip
 // overrides them).
 constexpr int TSTRIP = 4;
 constexpr int TSTRIP_FP = 2;
@@ -650,7 +651,7 @@ __device__ __forceinline__ int item_index(const ContractArgs& a, int bid, int nb
   return a.order ? bid : xcd_remap(bid, nblocks);
 }
 
-// One workgroup (8 waves, two per SIMD) owns a 16 x 16 (e, f) tile, one
+// FP32 phase contraction (T = float).  One workgroup (8 waves, two per SIMD) owns a 16 x 16 (e, f) tile, one
 // primary derivative, one block of 16 base momenta and one timeslice, and
 // sweeps all sites in chunks of 16:
 //   stage 1: wave w forms the Q tiles of sites SPW*w.. of the chunk on MFMA
@@ -729,7 +730,7 @@ __device__ __forceinline__ void contract_body(const c_t<T>* __restrict__ W, cons
   };
 
   acc_t A1[NBW], A2[NBW], A3[NBW], A4[NBW];
-  double D1[NBW][4], D2[NBW][4], D3[NBW][4], D4[NBW][4];  // FP64 cross-chunk sums (T = float)
+  double D1[NBW][4], D2[NBW][4], D3[NBW][4], D4[NBW][4];  // FP64 cross-chunk sums
   T zr[NBW], zi[NBW];
   double Zr[NBW], Zi[NBW];
 #pragma unroll
@@ -740,7 +741,7 @@ __device__ __forceinline__ void contract_body(const c_t<T>* __restrict__ W, cons
 #pragma unroll
     for (int r = 0; r < 4; ++r) D1[b][r] = D2[b][r] = D3[b][r] = D4[b][r] = 0;
   }
-  // FP32 form: Q_d[e,f,x] often carries a large site-independent part (for
+  // Q_d[e,f,x] often carries a large site-independent part (for
   // d = 0, |V_e(x)|^2 >= 0).  Stage 2 works on Q - c with c the mean over the
   // first chunk, and adds c * sum_x Phi_b(x) back in FP64, so FP32 rounding
   // scales with the fluctuation of Q rather than with its mean.
@@ -801,7 +802,7 @@ __device__ __forceinline__ void contract_body(const c_t<T>* __restrict__ W, cons
   load_phase(0);
   stage1(0, 0);
   __syncthreads();
-  if constexpr (sizeof(T) == 4) {
+  {
     const int n0 = min(SC, g.V3);
 #pragma unroll
     for (int b = 0; b < NBW; ++b) {
@@ -827,10 +828,8 @@ __device__ __forceinline__ void contract_body(const c_t<T>* __restrict__ W, cons
 #pragma unroll
       for (int b = 0; b < NBW; ++b) {
         c_t<T> qq = Qs[buf][4 * k + g4][NBW * wave + b][l16];
-        if constexpr (sizeof(T) == 4) {
-          qq.x = real_site ? qq.x - cr[b] : (T)0;
-          qq.y = real_site ? qq.y - ci[b] : (T)0;
-        }
+        qq.x = real_site ? qq.x - cr[b] : (T)0;
+        qq.y = real_site ? qq.y - ci[b] : (T)0;
         A1[b] = mfma<T>::mac(pr, qq.x, A1[b]);
         A2[b] = mfma<T>::mac(pi, qq.y, A2[b]);
         A3[b] = mfma<T>::mac(pi, qq.x, A3[b]);
@@ -841,40 +840,23 @@ __device__ __forceinline__ void contract_body(const c_t<T>* __restrict__ W, cons
     }
     if (c0 + SC < g.V3P) load_phase(c0 + SC);
 
-    if constexpr (sizeof(T) == 4) {
-      // FP32 partial sums of one chunk are moved into FP64 accumulators.
-#pragma unroll
-      for (int b = 0; b < NBW; ++b) {
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          D1[b][r] += (double)A1[b][r];
-          D2[b][r] += (double)A2[b][r];
-          D3[b][r] += (double)A3[b][r];
-          D4[b][r] += (double)A4[b][r];
-        }
-        A1[b] = A2[b] = A3[b] = A4[b] = acc_t{0, 0, 0, 0};
-        Zr[b] += (double)zr[b];
-        Zi[b] += (double)zi[b];
-        zr[b] = zi[b] = 0;
-      }
-    }
-    __syncthreads();
-  }
-  if constexpr (sizeof(T) == 8) {
+    // FP32 partial sums of one chunk are moved into FP64 accumulators.
 #pragma unroll
     for (int b = 0; b < NBW; ++b) {
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        D1[b][r] = (double)A1[b][r];
-        D2[b][r] = (double)A2[b][r];
-        D3[b][r] = (double)A3[b][r];
-        D4[b][r] = (double)A4[b][r];
+        D1[b][r] += (double)A1[b][r];
+        D2[b][r] += (double)A2[b][r];
+        D3[b][r] += (double)A3[b][r];
+        D4[b][r] += (double)A4[b][r];
       }
-      Zr[b] = (double)zr[b];
-      Zi[b] = (double)zi[b];
+      A1[b] = A2[b] = A3[b] = A4[b] = acc_t{0, 0, 0, 0};
+      Zr[b] += (double)zr[b];
+      Zi[b] += (double)zi[b];
+      zr[b] = zi[b] = 0;
     }
+    __syncthreads();
   }
-
   // ---- epilogue ----
   const int Ne = g.Ne, P = a.P;
   const size_t plane = (size_t)Ne * Ne;

@@ -137,6 +137,8 @@ int ed_compute(ed_context* ctx, int t0, int nt, int mode, void* out, int out_on_
  *     32) fails with ED_ERR_UNSUPPORTED.
  *   - the plan tables must be built: ed_compute or ed_query once after the
  *     last ed_set_* / ed_set_option call; otherwise ED_ERR_STATE.
+ *   - the FP64 form also keeps its x-y sums of up to eight timeslices (16 MiB, or
+ *     one timeslice's where that is more) in a buffer allocated with the plan.
  *   - nothing is allocated or freed and no event is recorded; the used part of
  *     the workspace is cleared by a fill kernel on each call (the workspace
  *     keeps the previous call's contents).
@@ -188,10 +190,12 @@ int ed_synchronize(ed_context* ctx);
  *                         ed_orthonormality only.
  *   ED_OPT_STRIP          tile order of the contraction: its 16 x 16 (e, f) tiles run in strips
  *                         of this many e-tile rows, f-tile by f-tile inside a strip (0, default:
- *                         4 for the mixed kernels, 2 for the FP64 / FP32 kernel).  Chosen by
- *                         ed_tune.
+ *                         4 for the mixed kernels, 2 for the FP64 / FP32 kernel; the FP64 kernel
+ *                         takes its tiles in blocks of 2 x 2 and rounds the height to 2, 4 or
+ *                         8).  Chosen by ed_tune.
  *   ED_OPT_ITEM_ORDER     contraction work items over the 8 XCDs: 0 (default) contiguous ranges
- *                         per XCD, 1 round robin.  Chosen by ed_tune.
+ *                         per XCD (FP64 kernel: runs of 32 items), 1 round robin.  Chosen by
+ *                         ed_tune.
  *   ED_OPT_H16_UNIT       1 (default): ED_OPT_MIXED_WS 2 runs the unit plan where it applies
  *                         (every split coefficient +1: the workspace stores each derivative
  *                         level k times i^k, splits of multiplicity m enter m times, results
@@ -243,7 +247,8 @@ int ed_profile_reset(ed_context* ctx);
 
 /* Plan figures for the current lattice / derivative / momentum settings
  * (used for roofline accounting; no counterpart in the reference):
- *   ED_Q_CONTRACT_FLOPS_PER_T  MFMA flops the contraction executes per timeslice
+ *   ED_Q_CONTRACT_FLOPS_PER_T  flops the FP64 contraction executes per timeslice (matrix split
+ *                              sum and vector sums over x; the y and z sums are left out)
  *   ED_Q_ALGO_FLOPS_PER_T      8 Ne^2 (3 V3) S P, the direct split-by-split
  *                              formulation (S = number of split terms)
  *   ED_Q_PRIMARY_DERIVATIVES   derivatives contracted (the others follow by
@@ -258,7 +263,7 @@ int ed_profile_reset(ed_context* ctx);
  *                              with uniform waves, 3 warp-specialized (32-bit workspace
  *                              offsets), 4 warp-specialized with 64-bit addresses, 5 FP16
  *                              stage 1
- * (ED_Q_CONTRACT_FLOPS_PER_T counts the FP64 / FP32-stage-2 kernels.) */
+ */
 enum ed_query {
   ED_Q_CONTRACT_FLOPS_PER_T = 1,
   ED_Q_ALGO_FLOPS_PER_T = 2,
