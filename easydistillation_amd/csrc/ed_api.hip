@@ -145,6 +145,8 @@ struct ed_context {
 
   DevBuf<double2> U64;
   DevBuf<float2> V;
+  DevBuf<unsigned long long> vstat;  // ed_set_eigvecs: largest component, orthonormality deviation
+  DevBuf<double2> gram;              // its sums over ranges of sites (at most 64 MB)
   DevBuf<double> wgt;
   bool use_wgt = false;
 
@@ -1022,64 +1024,150 @@ void build_plan(ed_context* c) {
   ++c->gen;
 }
 
-__global__ void c128_to_c64_kernel(const double2* __restrict__ in, float2* __restrict__ out, size_t n) {
-  for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x)
-    out[i] = make_float2((float)in[i].x, (float)in[i].y);
-}
-// largest |re|, |im| over n complex64 values into *m (bit pattern of a
-// non-negative float, so unsigned order is float order); *m starts at 0
-__global__ void absmax_c64_kernel(const float2* __restrict__ in, size_t n, unsigned int* __restrict__ m) {
+// n input values (complex64 or complex128) to complex64 at out, and their largest
+// |re|, |im| into *m (bit pattern of a non-negative float, so unsigned order is
+// float order); *m starts at 0.  out may be the input itself.  One pass over
+// HBM: copy and maximum apart took 84 + 41 us for 93 MB.
+template <typename IN>
+__global__ __launch_bounds__(256) void take_v_kernel(const IN* in, float2* out, size_t n, unsigned int* __restrict__ m) {
   float v = 0.f;
-  for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x)
-    v = fmaxf(v, fmaxf(fabsf(in[i].x), fabsf(in[i].y)));
+  const size_t stride = (size_t)gridDim.x * 256;
+  size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
+  auto take = [&](const IN w, size_t k) {
+    const float2 x = make_float2((float)w.x, (float)w.y);
+    out[k] = x;
+    v = fmaxf(v, fmaxf(fabsf(x.x), fabsf(x.y)));
+  };
+  for (; i + 3 * stride < n; i += 4 * stride) {
+    const IN w0 = in[i], w1 = in[i + stride], w2 = in[i + 2 * stride], w3 = in[i + 3 * stride];
+    take(w0, i), take(w1, i + stride), take(w2, i + 2 * stride), take(w3, i + 3 * stride);
+  }
+  for (; i < n; i += stride) take(in[i], i);
+  // one atomic per workgroup: one per wave (8192) took as long as the copy
+  __shared__ float wm[4];
   v = ed::wave_max_nonneg(v);
-  if ((threadIdx.x & 63) == 0) atomicMax(m, __float_as_uint(v));
+  if ((threadIdx.x & 63) == 0) wm[threadIdx.x >> 6] = v;
+  __syncthreads();
+  if (threadIdx.x == 0) atomicMax(m, __float_as_uint(fmaxf(fmaxf(wm[0], wm[1]), fmaxf(wm[2], wm[3]))));
 }
-// FP64 max |(V_t^dag V_t)[e][f] - delta_ef| over one 32 x 32 tile (e, f) of
-// timeslice t0 + blockIdx.z; each row of V_t holds K = 3 V3 complex64 values.
-// Products of complex64 values are exact in FP64 and the sums run in FP64.
-// The tile maximum is maxed into *dev as the bit pattern of a non-negative
-// double (unsigned order is double order); *dev starts at 0.
-__global__ __launch_bounds__(256) void gram_dev_kernel(const float2* __restrict__ V, int Ne, size_t K, int t0,
-                                                      unsigned long long* __restrict__ dev) {
-  constexpr int KC = 32;
-  __shared__ double2 A[32][KC + 1], B[32][KC + 1];
-  const int tid = threadIdx.x, tx = tid & 15, ty = tid >> 4;
-  const int e0 = blockIdx.x * 32, f0 = blockIdx.y * 32;
+
+// FP64 sums (V_t^dag V_t)[e][f] over one K range of one 64 x 64 tile, te <= tf (the
+// rest is the conjugate).  Each row of V_t holds K = 3 V3 complex64 values;
+// their products are exact in FP64 and the sums run in FP64 on the matrix units:
+// the floats of a row, real and imaginary parts in turn, are the real terms of
+// Re conj(a) b = ar br + ai bi; Im conj(a) b = ar bi - ai br takes the other
+// float of each pair of b with alternating sign.
+//
+// Bound: FP64 units (0.28 ms for 8 timeslices of 24^3, Nev 128 at 78 TF).  The
+// former vector kernel ran one workgroup per 32 x 32 tile and timeslice over all
+// of K (128 workgroups there) at 6.0 ms; K ranges fill the chip.
+//
+// With one range the largest |sum - delta_ef| is maxed into *dev (bit pattern of
+// a non-negative double, unsigned order is double order; *dev starts at 0);
+// otherwise the sums go to part[t][tile][range][64][64] for gram_max_kernel.
+constexpr int GR_T = 64, GR_K = 32, GR_P = 2 * GR_K + 4;  // tile, K chunk, floats per LDS row (banks 4 row + k: no conflict)
+__device__ __forceinline__ void gram_tile(int idx, int nt, int& te, int& tf) {
+  te = 0;
+  while (idx >= nt - te) idx -= nt - te++;
+  tf = te + idx;
+}
+__device__ __forceinline__ void gram_dev(double d, unsigned long long* dev) {
+  for (int off = 32; off > 0; off >>= 1) d = fmax(d, __shfl_xor(d, off));
+  if ((threadIdx.x & 63) == 0) atomicMax(dev, (unsigned long long)__double_as_longlong(d));
+}
+// grid (tiles te <= tf, ranges, timeslices), block 256: wave w takes rows 32 (w / 2), columns 32 (w mod 2)
+__global__ __launch_bounds__(256) void gram_kernel(const float2* __restrict__ V, int Ne, size_t K, size_t kpart, int t0,
+                                                   double2* __restrict__ part, unsigned long long* __restrict__ dev) {
+  typedef ed::mfma<double>::acc acc_t;
+  __shared__ float A[GR_T * GR_P], B[GR_T * GR_P];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l16 = lane & 15, g4 = lane >> 4;
+  int te, tf;
+  gram_tile(blockIdx.x, (Ne + GR_T - 1) / GR_T, te, tf);
+  const int e0 = te * GR_T, f0 = tf * GR_T;
   const float2* Vt = V + (size_t)(t0 + blockIdx.z) * Ne * K;
-  double re[2][2] = {{0.0, 0.0}, {0.0, 0.0}}, im[2][2] = {{0.0, 0.0}, {0.0, 0.0}};
-  for (size_t k0 = 0; k0 < K; k0 += KC) {
-    for (int i = tid; i < 32 * KC; i += 256) {
-      const int r = i / KC, k = i % KC;
-      const size_t kk = k0 + k;
-      float2 a = make_float2(0.f, 0.f), b = make_float2(0.f, 0.f);
-      if (kk < K) {
-        if (e0 + r < Ne) a = Vt[(size_t)(e0 + r) * K + kk];
-        if (f0 + r < Ne) b = Vt[(size_t)(f0 + r) * K + kk];
+  const size_t k0 = blockIdx.y * kpart, k1 = min(k0 + kpart, K);
+  constexpr int R = GR_T * GR_K / 256;  // values per thread, side and chunk
+  float2 ra[R], rb[R];
+  auto fetch = [&](size_t k) {
+#pragma unroll
+    for (int i = 0; i < R; ++i) {
+      const int r = (tid >> 5) + 8 * i;
+      const size_t kk = k + (tid & 31);
+      ra[i] = rb[i] = make_float2(0.f, 0.f);
+      if (kk < k1) {
+        if (e0 + r < Ne) ra[i] = Vt[(size_t)(e0 + r) * K + kk];
+        if (f0 + r < Ne) rb[i] = Vt[(size_t)(f0 + r) * K + kk];
       }
-      A[r][k] = make_double2(a.x, a.y);
-      B[r][k] = make_double2(b.x, b.y);
+    }
+  };
+  acc_t re[2][2], im[2][2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j) re[i][j] = im[i][j] = acc_t{0.0, 0.0, 0.0, 0.0};
+  const float sgn = g4 & 1 ? -1.f : 1.f;
+  const float* pa = A + (32 * (wave >> 1) + l16) * GR_P + g4;
+  const float* pb = B + (32 * (wave & 1) + l16) * GR_P + g4;
+  const float* pc = B + (32 * (wave & 1) + l16) * GR_P + (g4 ^ 1);
+  fetch(k0);
+  for (size_t k = k0; k < k1; k += GR_K) {
+    __syncthreads();  // the previous chunk is used up
+#pragma unroll
+    for (int i = 0; i < R; ++i) {
+      const int o = ((tid >> 5) + 8 * i) * GR_P + 2 * (tid & 31);
+      *(float2*)&A[o] = ra[i];
+      *(float2*)&B[o] = rb[i];
     }
     __syncthreads();
-    for (int k = 0; k < KC; ++k) {
-      const double2 a[2] = {A[ty][k], A[ty + 16][k]};
-      const double2 b[2] = {B[tx][k], B[tx + 16][k]};
+    if (k + GR_K < k1) fetch(k + GR_K);
+#pragma unroll 4
+    for (int s = 0; s < GR_K / 2; ++s) {
+      double a[2], b[2], c[2];
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        a[i] = (double)pa[16 * i * GR_P + 4 * s];
+        b[i] = (double)pb[16 * i * GR_P + 4 * s];
+        c[i] = (double)(sgn * pc[16 * i * GR_P + 4 * s]);
+      }
+#pragma unroll
       for (int i = 0; i < 2; ++i)
-        for (int j = 0; j < 2; ++j) {  // conj(a) b
-          re[i][j] += a[i].x * b[j].x + a[i].y * b[j].y;
-          im[i][j] += a[i].x * b[j].y - a[i].y * b[j].x;
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+          re[i][j] = ed::mfma<double>::mac(a[i], b[j], re[i][j]);
+          im[i][j] = ed::mfma<double>::mac(a[i], c[j], im[i][j]);
         }
     }
-    __syncthreads();
   }
   double d = 0.0;
+#pragma unroll
   for (int i = 0; i < 2; ++i)
-    for (int j = 0; j < 2; ++j) {
-      const int e = e0 + ty + 16 * i, f = f0 + tx + 16 * j;
-      if (e < Ne && f < Ne) d = fmax(d, hypot(re[i][j] - (e == f ? 1.0 : 0.0), im[i][j]));
-    }
-  for (int off = 32; off > 0; off >>= 1) d = fmax(d, __shfl_xor(d, off));
-  if ((tid & 63) == 0) atomicMax(dev, (unsigned long long)__double_as_longlong(d));
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int el = 32 * (wave >> 1) + 16 * i + ed::mfma<double>::row(g4, r), fl = 32 * (wave & 1) + 16 * j + l16;
+        if (part)
+          part[(((size_t)blockIdx.z * gridDim.x + blockIdx.x) * gridDim.y + blockIdx.y) * (GR_T * GR_T) + el * GR_T + fl] =
+              make_double2(re[i][j][r], im[i][j][r]);
+        else if (e0 + el < Ne && f0 + fl < Ne)
+          d = fmax(d, hypot(re[i][j][r] - (e0 + el == f0 + fl ? 1.0 : 0.0), im[i][j][r]));
+      }
+  if (!part) gram_dev(d, dev);
+}
+// grid (tiles, 16, timeslices), block 256: the ranges of 256 elements of a tile
+__global__ __launch_bounds__(256) void gram_max_kernel(const double2* __restrict__ part, int Ne, int nr,
+                                                       unsigned long long* __restrict__ dev) {
+  int te, tf;
+  gram_tile(blockIdx.x, (Ne + GR_T - 1) / GR_T, te, tf);
+  const int o = blockIdx.y * 256 + threadIdx.x, e = te * GR_T + o / GR_T, f = tf * GR_T + o % GR_T;
+  const double2* p = part + ((size_t)blockIdx.z * gridDim.x + blockIdx.x) * nr * (GR_T * GR_T) + o;
+  double re = 0.0, im = 0.0;
+  for (int k = 0; k < nr; ++k) {
+    const double2 v = p[(size_t)k * (GR_T * GR_T)];
+    re += v.x;
+    im += v.y;
+  }
+  gram_dev(e < Ne && f < Ne ? hypot(re - (e == f ? 1.0 : 0.0), im) : 0.0, dev);
 }
 
 __global__ void c64_to_c128_kernel(const float2* __restrict__ in, double2* __restrict__ out, size_t n) {
@@ -2011,21 +2099,33 @@ int ed_set_eigvecs(ed_context* ctx, const void* V, int dtype, int on_device) {
     HIPCHK(hipSetDevice(ctx->device));
     const size_t n = (size_t)ctx->Lt * ctx->Ne * ctx->V3 * 3;
     ctx->V.ensure(n);
-    if (dtype == ED_C64) {
-      HIPCHK(hipMemcpyAsync(ctx->V.p, V, n * sizeof(float2), on_device ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice,
-                            ctx->stream));
+    // [0] largest component of V, [1] largest deviation from orthonormality
+    ctx->vstat.ensure(2);
+    HIPCHK(hipMemsetAsync(ctx->vstat.p, 0, 2 * sizeof(unsigned long long), ctx->stream));
+    unsigned int* mx = (unsigned int*)(void*)ctx->vstat.p;
+    auto take = [&](const auto* in, float2* out, size_t m) {
+      const unsigned grid = (unsigned)std::min<size_t>(2048, (m + 1023) / 1024);
+      take_v_kernel<<<grid, 256, 0, ctx->stream>>>(in, out, m, mx);
+      HIPCHK(hipGetLastError());
+    };
+    if (dtype == ED_C64 && on_device) {
+      take((const float2*)V, ctx->V.p, n);
+    } else if (dtype == ED_C64) {
+      HIPCHK(hipMemcpyAsync(ctx->V.p, V, n * sizeof(float2), hipMemcpyHostToDevice, ctx->stream));
+      take(ctx->V.p, ctx->V.p, n);
+    } else if (on_device) {
+      // complex128 is rounded to complex64 (the reference's c8 staging buffer)
+      take((const double2*)V, ctx->V.p, n);
     } else {
-      // round complex128 to complex64 (the reference's c8 staging buffer)
       const size_t chunk = (size_t)1 << 24;
       DevBuf<double2> tmp;
       tmp.ensure(std::min(n, chunk));
       for (size_t s = 0; s < n; s += chunk) {
         const size_t m = std::min(chunk, n - s);
-        HIPCHK(hipMemcpyAsync(tmp.p, (const double2*)V + s, m * sizeof(double2),
-                              on_device ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice, ctx->stream));
-        c128_to_c64_kernel<<<1024, 256, 0, ctx->stream>>>(tmp.p, ctx->V.p + s, m);
-        HIPCHK(hipGetLastError());
+        HIPCHK(hipMemcpyAsync(tmp.p, (const double2*)V + s, m * sizeof(double2), hipMemcpyHostToDevice, ctx->stream));
+        take(tmp.p, ctx->V.p + s, m);
       }
+      HIPCHK(hipStreamSynchronize(ctx->stream));  // tmp is freed here
     }
     ctx->v64_set = false;
     if (ctx->exact_v) {
@@ -2041,43 +2141,43 @@ int ed_set_eigvecs(ed_context* ctx, const void* V, int dtype, int on_device) {
     } else {
       ctx->V64.reset();
     }
+    // FP64 orthonormality of the stored eigenvectors, every timeslice: ranges of
+    // K where the tiles alone give fewer than 1024 workgroups, at least 256 values
+    // each; their sums (64 KB per workgroup) stay below 64 MB
     {
-      // scale of the FP16 stage-1 workspace: from the largest component
-      DevBuf<unsigned int> mx;
-      mx.ensure(1);
-      HIPCHK(hipMemsetAsync(mx.p, 0, sizeof(unsigned int), ctx->stream));
-      absmax_c64_kernel<<<1024, 256, 0, ctx->stream>>>(ctx->V.p, n, mx.p);
-      HIPCHK(hipGetLastError());
-      unsigned int h = 0;
-      HIPCHK(hipMemcpyAsync(&h, mx.p, sizeof(h), hipMemcpyDeviceToHost, ctx->stream));
-      HIPCHK(hipStreamSynchronize(ctx->stream));
-      float f;
-      std::memcpy(&f, &h, sizeof(f));
-      if (!std::isfinite(f)) fail(ED_ERR_ARG, "eigenvectors hold a non-finite value");
-      ctx->vmax = f;
-    }
-    {
-      // FP64 orthonormality of the stored eigenvectors, every timeslice
-      DevBuf<unsigned long long> dv;
-      dv.ensure(1);
-      HIPCHK(hipMemsetAsync(dv.p, 0, sizeof(unsigned long long), ctx->stream));
       const size_t K = (size_t)3 * ctx->V3;
-      const unsigned nb = (unsigned)((ctx->Ne + 31) / 32);
+      const unsigned nt = (unsigned)((ctx->Ne + GR_T - 1) / GR_T), tiles = nt * (nt + 1) / 2;
+      const size_t all = (size_t)tiles * ctx->Lt;
+      const size_t want = std::max<size_t>(1, std::min<size_t>(1024 / all, K / 256));
+      const size_t kpart = ((K + want - 1) / want + GR_K - 1) / GR_K * GR_K;
+      const unsigned nr = (unsigned)((K + kpart - 1) / kpart);
+      if (nr > 1) ctx->gram.ensure(all * nr * GR_T * GR_T);
       for (int t0 = 0; t0 < ctx->Lt; t0 += 1024) {
         const unsigned nz = (unsigned)std::min(1024, ctx->Lt - t0);
-        gram_dev_kernel<<<dim3(nb, nb, nz), 256, 0, ctx->stream>>>(ctx->V.p, ctx->Ne, K, t0, dv.p);
+        gram_kernel<<<dim3(tiles, nr, nz), 256, 0, ctx->stream>>>(ctx->V.p, ctx->Ne, K, kpart, t0,
+                                                                  nr > 1 ? ctx->gram.p : nullptr, ctx->vstat.p + 1);
         HIPCHK(hipGetLastError());
+        if (nr > 1) {
+          gram_max_kernel<<<dim3(tiles, GR_T * GR_T / 256, nz), 256, 0, ctx->stream>>>(ctx->gram.p, ctx->Ne, (int)nr,
+                                                                                      ctx->vstat.p + 1);
+          HIPCHK(hipGetLastError());
+        }
       }
-      unsigned long long h = 0;
-      HIPCHK(hipMemcpyAsync(&h, dv.p, sizeof(h), hipMemcpyDeviceToHost, ctx->stream));
-      HIPCHK(hipStreamSynchronize(ctx->stream));
-      std::memcpy(&ctx->vv_dev, &h, sizeof(double));
-      ctx->eig_set = false;
-      if (ctx->ortho_gate > 0 && !(ctx->vv_dev <= std::pow(10.0, -ctx->ortho_gate)))
-        fail(ED_ERR_ARG, "eigenvectors are not orthonormal: max|V^dag V - 1| = %.3e > 1e-%d", ctx->vv_dev,
-             ctx->ortho_gate);
     }
+    unsigned long long stat[2];
+    HIPCHK(hipMemcpyAsync(stat, ctx->vstat.p, sizeof(stat), hipMemcpyDeviceToHost, ctx->stream));
     HIPCHK(hipStreamSynchronize(ctx->stream));
+    // scale of the FP16 stage-1 workspace: from the largest component
+    float f;
+    const unsigned int bits = (unsigned int)stat[0];
+    std::memcpy(&f, &bits, sizeof(f));
+    if (!std::isfinite(f)) fail(ED_ERR_ARG, "eigenvectors hold a non-finite value");
+    ctx->vmax = f;
+    std::memcpy(&ctx->vv_dev, &stat[1], sizeof(double));
+    ctx->eig_set = false;
+    if (ctx->ortho_gate > 0 && !(ctx->vv_dev <= std::pow(10.0, -ctx->ortho_gate)))
+      fail(ED_ERR_ARG, "eigenvectors are not orthonormal: max|V^dag V - 1| = %.3e > 1e-%d", ctx->vv_dev,
+           ctx->ortho_gate);
     ctx->eig_set = true;
   });
 }

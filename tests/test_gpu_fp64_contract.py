@@ -56,3 +56,19 @@ def test_fp64_contraction_against_oracle(latt, Ne, nabla, moms):
     g1.load_arrays(U, V)
     t = latt[3] - 1
     assert np.array_equal(g1.calc_range(t, 1)[0], E[t])
+
+
+@pytest.mark.parametrize("latt,Ne", [([3, 3, 3, 1], 1), ([4, 4, 5, 3], 63), ([4, 4, 5, 2], 64), ([5, 7, 9, 2], 65),
+                                     ([6, 6, 6, 1], 130), ([16, 16, 16, 1], 70)])
+@pytest.mark.parametrize("dtype", [np.complex64, np.complex128])
+def test_orthonormality_of_uneven_blocks(latt, Ne, dtype):
+    """max|V^dag V - 1| over 64 x 64 tiles and ranges of sites, one eigenvector off by 1e-3."""
+    rng = np.random.default_rng(Ne)
+    V = S.eigvecs_np(rng, latt, Ne)
+    V[latt[3] - 1, Ne - 1] *= np.float32(1.001)
+    g = ed.ElementalGenerator(latt, None, None, 0, [(0, 0, 0)], Ne=Ne)
+    g.load_arrays(S.gauge_np(rng, latt, "unit"), V.astype(dtype))
+    W = V.astype(np.complex128).reshape(latt[3], Ne, -1)
+    want = max(np.abs(w.conj() @ w.T - np.eye(Ne)).max() for w in W)
+    # both sum products of complex64 values in FP64: K terms of at most 1, 1e-16 each
+    assert abs(g.context.orthonormality() - want) <= 1e-13
