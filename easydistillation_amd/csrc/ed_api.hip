@@ -208,9 +208,8 @@ struct ed_context {
   int64_t f_macs = 0;               // multiply-adds of one timeslice
   DevBuf<char> ftab;                // axis functions, then MomTerm, Group and slot tables
   size_t f_mt = 0, f_grp = 0, f_slot = 0;  // byte offsets of the last three
-  DevBuf<double> M;                 // moments of a batch
-  DevBuf<double> Mfix;              // moments of ed_compute_noalloc, allocated with the plan
-  int fix_tb = 0;                   // timeslices Mfix holds
+  DevBuf<double> M;                 // x-y sums of a batch of timeslices
+  DevBuf<double> Mfix;              // one timeslice's for ed_compute_noalloc where its workspace has no room
 
   // reverse pass
   int bns_max = 1;        // largest merged split count of one derivative
@@ -1009,17 +1008,14 @@ void build_plan(ed_context* c) {
     HIPCHK(hipMemcpy(c->phase_grp.p, pa.data(), pa.size() * sizeof(double2), hipMemcpyHostToDevice));
     HIPCHK(hipMemcpy(c->child_of.p, child.data(), child.size() * sizeof(int), hipMemcpyHostToDevice));
   }
-  // moments of ed_compute_noalloc, which cannot allocate: up to eight
-  // timeslices within 16 MiB, at least one, for lattices its workspace holds
-  c->fix_tb = 0;
-  if ((size_t)c->slots() * c->NeP * 3 * c->V3P * sizeof(double2) <= ED_NOALLOC_SCRATCH_BYTES) {
-    const size_t per_t = moments_per_t(c);
-    const size_t n = std::max<size_t>(1, std::min<size_t>({(size_t)8, (size_t)c->Lt, ((size_t)2 << 20) / per_t}));
-    c->Mfix.ensure(n * per_t);
-    c->fix_tb = (int)n;
-  } else {
+  // x-y sums of ed_compute_noalloc, which cannot allocate: behind the displaced
+  // vectors in its fixed workspace, or, for lattices that leave no room there, one
+  // timeslice's allocated with the plan
+  const size_t ws1 = (size_t)c->slots() * c->NeP * 3 * c->V3P * sizeof(double2), m1 = moments_per_t(c) * sizeof(double);
+  if (ws1 <= ED_NOALLOC_SCRATCH_BYTES && ws1 + m1 > ED_NOALLOC_SCRATCH_BYTES)
+    c->Mfix.ensure(moments_per_t(c));
+  else
     c->Mfix.reset();
-  }
   c->plan_dirty = false;
   ++c->gen;
 }
@@ -1376,15 +1372,17 @@ void run_batches(ed_context* c, int t0, int nt, double2* out_dev, void* out_host
   const bool noalloc = fixed != nullptr;
   int TB;
   ed::c_t<T>* W;
+  double* Mf = nullptr;  // x-y sums of the FP64 form
   if (noalloc) {
     const size_t per_t = per_t_ws_bytes<T>(c);
     if (per_t > fixed_bytes)
       fail(ED_ERR_UNSUPPORTED,
            "one timeslice needs %zu bytes of workspace; the no-allocation entry point holds at most %zu "
            "(use ed_compute)", per_t, fixed_bytes);
-    TB = std::min<int>(nt, (int)std::min<size_t>(fixed_bytes / per_t, (size_t)nt));
+    const size_t mom = sizeof(T) == 8 ? moments_per_t(c) * sizeof(double) : 0;
+    TB = (int)std::min<size_t>(std::max<size_t>(1, fixed_bytes / (per_t + mom)), (size_t)nt);
     if (c->tbatch_opt > 0) TB = std::min(TB, c->tbatch_opt);
-    if (sizeof(T) == 8) TB = std::min(TB, c->fix_tb);
+    Mf = (per_t + mom) * TB <= fixed_bytes ? (double*)(void*)(fixed + per_t * TB) : c->Mfix.p;
     W = (ed::c_t<T>*)(void*)fixed;
     const size_t n16 = per_t * TB / sizeof(uint4);
     zero_fill_kernel<<<(unsigned)std::min<size_t>(4096, (n16 + 255) / 256), 256, 0, c->stream>>>((uint4*)(void*)fixed,
@@ -1393,7 +1391,10 @@ void run_batches(ed_context* c, int t0, int nt, double2* out_dev, void* out_host
   } else {
     TB = auto_tbatch<T>(c, nt);
     W = ensure_workspace<T>(c, TB);
-    if (sizeof(T) == 8) c->M.ensure(moments_per_t(c) * TB);
+    if (sizeof(T) == 8) {
+      c->M.ensure(moments_per_t(c) * TB);
+      Mf = c->M.p;
+    }
   }
   const size_t out_t = (size_t)c->D * (c->moms.size() / 3) * c->Ne * c->Ne;
 
@@ -1415,7 +1416,7 @@ void run_batches(ed_context* c, int t0, int nt, double2* out_dev, void* out_host
     const int nb = std::min(TB, t0 + nt - tb0);
     if constexpr (sizeof(T) == 8) {
       enqueue_stencil<T>(c, W, tb0, nb, c->stream, launch);
-      enqueue_fp64(c, W, nb, out_dev ? (tb0 - t0) : 0, out, noalloc ? c->Mfix.p : c->M.p, c->stream, launch);
+      enqueue_fp64(c, W, nb, out_dev ? (tb0 - t0) : 0, out, Mf, c->stream, launch);
     } else {
     ContractArgs a = contract_args(c, nb, out_dev ? (tb0 - t0) : 0);
     const int nblk = (a.nwork + 7) / 8 * 8;

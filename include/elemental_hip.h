@@ -137,8 +137,8 @@ int ed_compute(ed_context* ctx, int t0, int nt, int mode, void* out, int out_on_
  *     32) fails with ED_ERR_UNSUPPORTED.
  *   - the plan tables must be built: ed_compute or ed_query once after the
  *     last ed_set_* / ed_set_option call; otherwise ED_ERR_STATE.
- *   - the FP64 form also keeps its x-y sums of up to eight timeslices (16 MiB, or
- *     one timeslice's where that is more) in a buffer allocated with the plan.
+ *   - the FP64 form keeps its x-y sums there too; where one timeslice's do not fit
+ *     behind its displaced vectors, in a buffer allocated with the plan.
  *   - nothing is allocated or freed and no event is recorded; the used part of
  *     the workspace is cleared by a fill kernel on each call (the workspace
  *     keeps the previous call's contents).
