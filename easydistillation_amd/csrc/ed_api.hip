@@ -2625,9 +2625,21 @@ int ed_laplacian(ed_context* ctx, int t, const void* F, void* out, int nvec, int
       dst = hout.p;
     }
     const ed::gauge::Lat L{ctx->Lx, ctx->Ly, ctx->Lz, ctx->Lt};
-    const size_t threads = (size_t)nvec * ctx->V3;
-    ed::gauge::laplacian_kernel<<<(unsigned)((threads + 255) / 256), 256, 0, ctx->stream>>>(src, dst, ctx->U64.p, L, t,
-                                                                                          nvec);
+    // vectors per thread: the links are read once for them all, so as many as
+    // still leave four workgroups of 256 sites per CU; below 4096 (vector, site
+    // block) pairs the chip is not filled by four per thread (latency of one
+    // thread's chain of neighbour loads), and each vector gets its own threads.
+    // 24^3 x 160 vectors (8640 pairs): 132 us with 8 per thread, 131 with 4,
+    // 202 with 2, 506 with one.
+    const size_t nb = ((size_t)ctx->V3 + 255) / 256;
+    auto go = [&](auto nv) {
+      constexpr int NV = decltype(nv)::value;
+      const size_t n = nb * ((nvec + NV - 1) / NV);
+      ed::gauge::laplacian_kernel<NV><<<(unsigned)((n + 7) / 8 * 8), 256, 0, ctx->stream>>>(src, dst, ctx->U64.p, L, t, nvec);
+    };
+    if (nb * nvec >= 8 * 1024) go(std::integral_constant<int, 8>{});
+    else if (nb * nvec >= 4 * 1024) go(std::integral_constant<int, 4>{});
+    else go(std::integral_constant<int, 1>{});
     HIPCHK(hipGetLastError());
     if (!on_device) {
       HIPCHK(hipMemcpyAsync(out, dst, n * sizeof(double2), hipMemcpyDeviceToHost, ctx->stream));

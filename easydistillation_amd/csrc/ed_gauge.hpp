@@ -268,45 +268,67 @@ __global__ __launch_bounds__(256) void polar_step_kernel(const double2* __restri
 // 3-D gauge-covariant Laplacian on a block of vectors of timeslice t
 // (lattice/generator/eigenvector.py:11-26):
 //   (L F)(x) = 6 F(x) - sum_mu [U_mu(x) F(x + mu) + U_mu(x - mu)^dag F(x - mu)]
-// F and out [nvec][V3][3] complex128; one thread per (vector, site), sites
+// F and out [nvec][V3][3] complex128; one thread per site and NV vectors, sites
 // fastest so neighbouring threads read neighbouring 48-byte site vectors.
+//
+// Bound: HBM, F and out once (47 us for 160 vectors of 24^3 at the 4.5 TB/s of a
+// copy).  One thread per (vector, site) read the 864 bytes of links for every
+// 96 bytes of vectors; here they are in registers for NV vectors.  Each XCD gets
+// a contiguous range of (vector group, site block), so the planes a site's
+// neighbours lie in stay in its L2 (132 us against 142 without).  Measured at
+// that size, the call: 525 us before, 132 us now.  What is left is the latency
+// of the neighbour loads at two waves per SIMD: both directions' links in
+// registers, for twice the loads in flight, beat one direction at a time at
+// three waves (132 against 175 us).
+template <int NV>
 __global__ __launch_bounds__(256) void laplacian_kernel(const double2* __restrict__ F, double2* __restrict__ out,
                                                         const double2* __restrict__ U, Lat L, int t, int nvec) {
-  const size_t V3 = (size_t)L.Lx * L.Ly * L.Lz;
-  const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= V3 * (size_t)nvec) return;
-  const size_t e = i / V3;
-  const int s = (int)(i % V3);
+  const int V3 = L.Lx * L.Ly * L.Lz;
+  const unsigned nb = (V3 + 255) / 256, n = gridDim.x;  // n = 8 k: item k (b mod 8) + b / 8
+  const unsigned item = (blockIdx.x & 7) * (n >> 3) + (blockIdx.x >> 3);
+  const unsigned grp = item / nb;
+  const int s = (int)(item - grp * nb) * 256 + threadIdx.x, v0 = (int)grp * NV;
+  if (s >= V3 || v0 >= nvec) return;
+  const int nv = min(NV, nvec - v0);
   const int x = s % L.Lx, y = (s / L.Lx) % L.Ly, z = s / (L.Lx * L.Ly);
-  const double2* Fe = F + e * V3 * 3;
-  double2 acc[3];
+  const size_t vec = (size_t)V3 * 3;
+  const double2* F0 = F + (size_t)v0 * vec;
+  double2 acc[NV][3];
 #pragma unroll
-  for (int a = 0; a < 3; ++a) acc[a] = cscale(Fe[(size_t)s * 3 + a], 6.0);
+  for (int v = 0; v < NV; ++v)
+    if (v < nv) {
 #pragma unroll
+      for (int a = 0; a < 3; ++a) acc[v][a] = cscale(F0[v * vec + (size_t)s * 3 + a], 6.0);
+    }
+#pragma unroll 1
   for (int mu = 0; mu < 3; ++mu) {
     int fx = x, fy = y, fz = z, bx = x, by = y, bz = z;
     step(mu, +1, fx, fy, fz, L);
     step(mu, -1, bx, by, bz, L);
-    const size_t sf = ((size_t)fz * L.Ly + fy) * L.Lx + fx, sb = ((size_t)bz * L.Ly + by) * L.Lx + bx;
-    const double2* uf = U + 9 * L.link(mu, t, x, y, z);
-    const double2* ub = U + 9 * L.link(mu, t, bx, by, bz);
-    double2 pf[3], pb[3];
+    const double2* qf = F0 + (((size_t)fz * L.Ly + fy) * L.Lx + fx) * 3;
+    const double2* qb = F0 + (((size_t)bz * L.Ly + by) * L.Lx + bx) * 3;
+    const M3 uf = load_m3(U + 9 * L.link(mu, t, x, y, z)), ub = load_m3(U + 9 * L.link(mu, t, bx, by, bz));
 #pragma unroll
-    for (int b = 0; b < 3; ++b) {
-      pf[b] = Fe[sf * 3 + b];
-      pb[b] = Fe[sb * 3 + b];
-    }
+    for (int v = 0; v < NV; ++v)
+      if (v < nv) {
+        const double2 pf[3] = {qf[v * vec], qf[v * vec + 1], qf[v * vec + 2]};
+        const double2 pb[3] = {qb[v * vec], qb[v * vec + 1], qb[v * vec + 2]};
 #pragma unroll
-    for (int a = 0; a < 3; ++a)
+        for (int a = 0; a < 3; ++a)
 #pragma unroll
-      for (int b = 0; b < 3; ++b) {
-        acc[a] = csub(acc[a], cmul(uf[a * 3 + b], pf[b]));
-        acc[a] = csub(acc[a], ccmul(ub[b * 3 + a], pb[b]));  // (U^dag)_{ab} = conj(U_{ba})
+          for (int b = 0; b < 3; ++b) {
+            acc[v][a] = csub(acc[v][a], cmul(uf.a[a * 3 + b], pf[b]));
+            acc[v][a] = csub(acc[v][a], ccmul(ub.a[b * 3 + a], pb[b]));  // (U^dag)_{ab} = conj(U_{ba})
+          }
       }
   }
-  double2* o = out + e * V3 * 3 + (size_t)s * 3;
 #pragma unroll
-  for (int a = 0; a < 3; ++a) o[a] = acc[a];
+  for (int v = 0; v < NV; ++v)
+    if (v < nv) {
+      double2* o = out + (size_t)(v0 + v) * vec + (size_t)s * 3;
+#pragma unroll
+      for (int a = 0; a < 3; ++a) o[a] = acc[v][a];
+    }
 }
 
 }  // namespace gauge
