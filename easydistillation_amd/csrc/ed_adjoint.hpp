@@ -126,7 +126,7 @@ __global__ __launch_bounds__(256) void adj_transpose_kernel(const double2* __res
 
 struct AdjArgs {
   Geom g;
-  int D, Q;
+  int D, Q, nb;
 };
 
 // --------------------------------------------------------------------------
@@ -142,28 +142,44 @@ struct AdjArgs {
 // S, D are the same for the whole wave: GC groups at a time are read with
 // scalar loads issued together (the group count is padded to a multiple of
 // GC with zero groups).  The phases c_q(x), s_q(x) and the W values are per
-// lane, coalesced over consecutive sites; each W load serves RB rows and is
-// issued one f ahead.  With QR > 0 the group count is exactly QR and every
+// lane, coalesced over consecutive sites; each W load serves RB rows.  With
+// QR > 0 the group count is exactly QR and every
 // group's phases stay in registers; QR = 0 takes any multiple of GC and
 // reloads the phases of groups past the first chunk.
 // Every gWT element a thread updates is its own (its site, the wave's rows):
 // no atomics.  phase [Q][V3P] (zero on padded sites and groups).  WT, gWT:
 // per timeslice [nW][NeP][V3P][3].  B: per timeslice [D][Q][2][Ne][NeP].
-// grid (ceil(V3P / 256), NeP / RB, TB), block 256
+//
+// Bound: FP64 instruction rate, 13.6 ms for 24^3 x 8, Ne 128, num_nabla 1 and
+// seven momenta; what it waits for is the latency of the scalar loads (two
+// chunks per f) and of W.  The four waves of a workgroup take 16 consecutive
+// rows at the same 64 sites, so one read of W from the L2 serves four waves,
+// and consecutive workgroups of an XCD take the other rows at those sites
+// (44.6 -> 41.5 ms there; four waves at the same rows and 256 sites: 35.7 ms
+// against 32.5 of this kernel).  Up to two terms a split the kernel keeps to
+// 168 registers, three waves per SIMD, which hides more than W loads one f
+// ahead at two (32.5 against 41.5 ms).  Two rows per wave at four waves per
+// SIMD: 44 ms; one group per chunk: 38.5 ms.
+// grid: 8 ceil(ceil(V3P / 64) (NeP / 4 RB) TB / 8), block 256
 // --------------------------------------------------------------------------
 template <int NS, int RB, int GC, int QR>
-__global__ __launch_bounds__(256) void adj_contract_kernel(const double2* __restrict__ WT, double2* __restrict__ gWT,
+__global__ __launch_bounds__(256, NS <= 2 ? 3 : 1) void adj_contract_kernel(const double2* __restrict__ WT,
+                                                           double2* __restrict__ gWT,
                                                            const double2* __restrict__ Brow,
                                                            const double2* __restrict__ Bcol,
                                                            const double2* __restrict__ phase,
                                                            const SplitTerm* __restrict__ splits,
                                                            const int2* __restrict__ dsplit, AdjArgs a) {
   const int V3P = a.g.V3P, NeP = a.g.NeP, Ne = a.g.Ne, Q = a.Q;  // Q: a multiple of GC
-  const int x = blockIdx.x * 256 + threadIdx.x;
+  const unsigned n = gridDim.x, item = (blockIdx.x & 7) * (n >> 3) + (blockIdx.x >> 3);
+  const int nrg = NeP / (4 * RB), nsb = (V3P + 63) / 64;  // NeP: a multiple of 16
+  const int tb = item / (nrg * nsb);
+  if (tb >= a.nb) return;
+  const int sb = (item - tb * nrg * nsb) / nrg;
+  const int r0 = __builtin_amdgcn_readfirstlane((item % nrg * 4 + (threadIdx.x >> 6)) * RB);  // < NeP
+  const int x = sb * 64 + (threadIdx.x & 63);
   const bool live = x < V3P;
   const int xc = live ? x : 0;
-  const int r0 = blockIdx.y * RB;  // < NeP
-  const int tb = blockIdx.z;
   const size_t rowsz = (size_t)V3P * 3;  // one row of one slot
   const size_t slotsz = (size_t)NeP * rowsz;
   const double2* Wb = WT + (size_t)tb * a.g.nW * slotsz + (size_t)xc * 3;
@@ -191,20 +207,13 @@ __global__ __launch_bounds__(256) void adj_contract_kernel(const double2* __rest
         for (int k = 0; k < NS; ++k)
 #pragma unroll
           for (int c = 0; c < 3; ++c) acc[i][k][c] = make_double2(0.0, 0.0);
-      double2 wn[NS][3];  // W of the next f
-#pragma unroll
-      for (int k = 0; k < NS; ++k)
-#pragma unroll
-        for (int c = 0; c < 3; ++c) wn[k][c] = src[k][c];
       for (int f = 0; f < Ne; ++f) {
         double2 w[NS][3];
-        const int fn = min(f + 1, Ne - 1);
 #pragma unroll
         for (int k = 0; k < NS; ++k)
 #pragma unroll
           for (int c = 0; c < 3; ++c) {
-            w[k][c] = wn[k][c];
-            wn[k][c] = src[k][(size_t)fn * rowsz + c];
+            w[k][c] = src[k][(size_t)f * rowsz + c];
           }
         double2 gam[RB];
 #pragma unroll

@@ -1572,13 +1572,14 @@ void run_backward(ed_context* c, int t0, int nt, const double2* G, bool g_dev, d
     a.g = g;
     a.D = D;
     a.Q = c->nq;
+    a.nb = nb;
     c->launch(ED_KERNEL_ADJOINT, [&] {
       int rb, gc;
       adj_shape(c->bns_max, rb, gc);
       auto go = [&](auto ns, auto rbc) {
         constexpr int NS = decltype(ns)::value, RB = decltype(rbc)::value;
         constexpr int GC = 8 / RB > 4 ? 4 : 8 / RB;
-        dim3 grid((c->V3P + 255) / 256, c->NeP / RB, nb);
+        const unsigned grid = ((c->V3P + 63) / 64 * (c->NeP / (4 * RB)) * nb + 7) / 8 * 8;
         const double2* const Wp = c->bWT.p;
         double2* const gp = c->bgWT.p;
         if (c->nq == 4)
