@@ -6,7 +6,8 @@ call (lattice/generator/elemental.py:290-338) and its callers loop
 ``ElementalGenerator`` instances -- lattices of different size, Ne, momenta
 and derivative depth -- and computes every timeslice of all of them with one
 replay of a captured hipGraph: per lattice the staging and hop kernels, then
-one persistent grouped contraction over the work of every lattice.  The
+one persistent grouped contraction over the work of every mixed lattice (an
+FP64 lattice runs its own).  The
 launch shape and work order are picked by the library's autotuner
 (``tune``).
 """

@@ -1693,8 +1693,8 @@ int guard(ed_context* ctx, const std::function<void()>& body) {
 // ---------------------------------------------------------------------------
 // Batched form: several contexts (lattices of different size and Ne) computed
 // by one stream-ordered sequence -- per lattice the staging and hop kernels
-// over all its timeslices, then one persistent grouped contraction per kernel
-// kind over every lattice -- captured once into a hipGraph and replayed with a
+// over all its timeslices, then one contraction per FP64 lattice and one
+// persistent grouped contraction per mixed kernel kind -- captured once into a hipGraph and replayed with a
 // single launch.
 // ---------------------------------------------------------------------------
 struct ed_batch {

@@ -330,7 +330,8 @@ int ed_get_gauge(ed_context* ctx, void* U, int on_device);
  * lattices of different size, Ne, momenta and derivative depth, each with its
  * inputs set -- computed together.  One run enqueues, for every context, the
  * staging and hop kernels over all its timeslices and then one persistent,
- * grouped contraction launch over the work items of every context; with
+ * grouped contraction launch over the work items of every mixed context (an
+ * FP64 one runs its own contraction over all its timeslices); with
  * ED_BOPT_GRAPH = 1 (default) this sequence is captured once into a hipGraph
  * and each run is a single graph launch (recaptured automatically when a
  * context's inputs, plan or buffers change).  Each context holds the
@@ -353,7 +354,8 @@ int ed_get_gauge(ed_context* ctx, void* U, int on_device);
  *                 reps runs each, keeps the fastest and returns its time. */
 typedef struct ed_batch ed_batch;
 enum ed_batch_option {
-  ED_BOPT_GRID_PER_CU = 1, /* persistent workgroups per CU (0: one per work item; default 2) */
+  ED_BOPT_GRID_PER_CU = 1, /* persistent workgroups per CU (0: one per work item; default 2);
+                              no effect on FP64 members                                     */
   ED_BOPT_ORDER = 2,       /* 0: contiguous item ranges per XCD (default), 1: round robin     */
   ED_BOPT_GRAPH = 3,       /* 1: capture and replay a hipGraph (default), 0: direct launches  */
   ED_BOPT_STRIP = 4,       /* tile-order strip height for every member (0: each context's own) */
