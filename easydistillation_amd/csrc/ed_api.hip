@@ -122,6 +122,12 @@ struct DevBuf {
   ~DevBuf() { reset(); }
 };
 
+// Part of a DevBuf that holds several tables.
+template <class T>
+struct DevView {
+  T* p = nullptr;
+};
+
 }  // namespace
 
 struct ed_context {
@@ -164,8 +170,9 @@ struct ed_context {
   int nsplit_max = 1;                 // largest merged split-term count over primary d
   int64_t h16_groups_sum[2] = {0, 0};         // sum of FP16 stage-1 k-groups
   float cmax = 1.f;                   // largest |split coefficient|
-  DevBuf<DPlan> dplan;
-  DevBuf<SplitTerm> splits;
+  DevBuf<char> tabs;  // the plan's small tables, one allocation and one copy: the views below
+  DevView<DPlan> dplan;
+  DevView<SplitTerm> splits;
   // unit plan of the FP16 stage-1 kernel (build_plan): every coefficient +1
   int h16_unit_opt = 1;               // ED_OPT_H16_UNIT
   int hop_lds = -1;                   // ED_OPT_HOP_LDS: the LDS-staged hop where the shape allows
@@ -175,8 +182,8 @@ struct ed_context {
   int64_t h16u_groups_sum[2] = {0, 0};
   DevBuf<DPlan> dplan_u;
   DevBuf<SplitTerm> splits_u;
-  DevBuf<int> pidx;  // plus [npb*16] then minus [npb*16]
-  DevBuf<double> psum;  // [npb*16] sum over sites of Phi_b
+  DevView<int> pidx;  // plus [npb*16] then minus [npb*16]
+  DevView<double> psum;  // [npb*16] sum over sites of Phi_b
   DevBuf<float> ph32;
   DevBuf<ed::half8> ph16;  // [npb][V3P/32][4][16][32] fp16 hi/lo of 2^14 Phi
   int mixed_stage2 = -1;   // 1: FP16 three-term split, 0: FP32 MFMA, -1: FP16 from V3 >= 4096 on
@@ -214,12 +221,12 @@ struct ed_context {
   // reverse pass
   int bns_max = 1;        // largest merged split count of one derivative
   int nparent_all = 0;    // slots that have children (levels below num_nabla)
-  DevBuf<SplitTerm> bsplits;
-  DevBuf<int2> bdsplit;
+  DevView<SplitTerm> bsplits;
+  DevView<int2> bdsplit;
   int nq = 0;                 // momentum groups: opposite pairs and single momenta
-  DevBuf<int2> bgroups;       // [nq] (p1, p2 or -1)
+  DevView<int2> bgroups;      // [nq] (p1, p2 or -1)
   DevBuf<double2> phase_grp;  // [nq][V3P] Phi of each group's first momentum (0 on padded sites)
-  DevBuf<int> child_of;       // [nparent_all][3]
+  DevView<int> child_of;      // [nparent_all][3]
   DevBuf<double2> bW, bA, bG, bOutV, bOutU;
   // W transposed to [slot][row][site][colour] for the contraction adjoint; the
   // same buffer then receives the gradient of W back in W's layout
@@ -919,16 +926,22 @@ void build_plan(ed_context* c) {
       HIPCHK(hipMemcpy(c->splits_u.p, spu.data(), spu.size() * sizeof(SplitTerm), hipMemcpyHostToDevice));
     }
   }
-  c->dplan.ensure(dpl.size());
-  c->splits.ensure(std::max<size_t>(1, sp.size()));
-  c->pidx.ensure(idx.size());
-  c->psum.ensure(ps.size());
+  // the small tables together: every allocation and every copy is a round trip
+  // of 10 to 20 us, which a new context of 4^3 x 8, Ne 20 waits for
+  std::vector<char> tabs;
+  std::vector<std::function<void()>> views;
+  auto put = [&](auto& view, const auto& v) {
+    const size_t at = (tabs.size() + 15) / 16 * 16, bytes = v.size() * sizeof(v[0]);
+    tabs.resize(at + bytes);
+    if (bytes) std::memcpy(tabs.data() + at, v.data(), bytes);
+    views.push_back([c, &view, at] { view.p = (std::remove_reference_t<decltype(view.p)>)(void*)(c->tabs.p + at); });
+  };
+  put(c->dplan, dpl);
+  put(c->splits, sp);
+  put(c->pidx, idx);
+  put(c->psum, ps);
   c->ph32.ensure(2 * pr.size());
   c->ph16.ensure(p16.size() / 8);
-  HIPCHK(hipMemcpy(c->dplan.p, dpl.data(), dpl.size() * sizeof(DPlan), hipMemcpyHostToDevice));
-  if (!sp.empty()) HIPCHK(hipMemcpy(c->splits.p, sp.data(), sp.size() * sizeof(SplitTerm), hipMemcpyHostToDevice));
-  HIPCHK(hipMemcpy(c->pidx.p, idx.data(), idx.size() * sizeof(int), hipMemcpyHostToDevice));
-  HIPCHK(hipMemcpy(c->psum.p, ps.data(), ps.size() * sizeof(double), hipMemcpyHostToDevice));
   HIPCHK(hipMemcpy(c->ph32.p, pr32.data(), pr32.size() * sizeof(float), hipMemcpyHostToDevice));
   HIPCHK(hipMemcpy(c->ph32.p + pr32.size(), pi32.data(), pi32.size() * sizeof(float), hipMemcpyHostToDevice));
   HIPCHK(hipMemcpy(c->ph16.p, p16.data(), p16.size() * sizeof(_Float16), hipMemcpyHostToDevice));
@@ -997,17 +1010,16 @@ void build_plan(ed_context* c) {
         t.push_back(mu);
         child[3 * pnt + mu] = derivative_index(t);
       }
-    c->bsplits.ensure(bsp.size());
-    c->bdsplit.ensure(bds.size());
-    c->bgroups.ensure(grp.size());
+    put(c->bsplits, bsp);
+    put(c->bdsplit, bds);
+    put(c->bgroups, grp);
+    put(c->child_of, child);
     c->phase_grp.ensure(pa.size());
-    c->child_of.ensure(child.size());
-    HIPCHK(hipMemcpy(c->bsplits.p, bsp.data(), bsp.size() * sizeof(SplitTerm), hipMemcpyHostToDevice));
-    HIPCHK(hipMemcpy(c->bdsplit.p, bds.data(), bds.size() * sizeof(int2), hipMemcpyHostToDevice));
-    HIPCHK(hipMemcpy(c->bgroups.p, grp.data(), grp.size() * sizeof(int2), hipMemcpyHostToDevice));
     HIPCHK(hipMemcpy(c->phase_grp.p, pa.data(), pa.size() * sizeof(double2), hipMemcpyHostToDevice));
-    HIPCHK(hipMemcpy(c->child_of.p, child.data(), child.size() * sizeof(int), hipMemcpyHostToDevice));
   }
+  c->tabs.ensure(tabs.size());
+  HIPCHK(hipMemcpy(c->tabs.p, tabs.data(), tabs.size(), hipMemcpyHostToDevice));
+  for (auto& view : views) view();
   // x-y sums of ed_compute_noalloc, which cannot allocate: behind the displaced
   // vectors in its fixed workspace, or, for lattices that leave no room there, one
   // timeslice's allocated with the plan
