@@ -171,7 +171,7 @@ struct ed_context {
   int64_t h16_groups_sum[2] = {0, 0};         // sum of FP16 stage-1 k-groups
   float cmax = 1.f;                   // largest |split coefficient|
   DevBuf<char> tabs;  // the plan's small tables, one allocation and one copy: the views below
-  DevView<DPlan> dplan;
+  DevView<DPlan> dplan, dplan64;
   DevView<SplitTerm> splits;
   // unit plan of the FP16 stage-1 kernel (build_plan): every coefficient +1
   int h16_unit_opt = 1;               // ED_OPT_H16_UNIT
@@ -601,7 +601,7 @@ void plan_fp64(ed_context* c, std::vector<DPlan>& dpl) {
   c->f_gt = 0;
   c->f_macs = 0;
   for (DPlan& p : dpl) {
-    p.grp0 = c->f_gt;
+    p.item0 = c->f_gt;
     c->f_gt += c->f_ngrp[0][p.mirror];
     const int64_t tiles = p.mirror ? nt * (nt + 1) / 2 : nt * nt;
     for (auto& b : c->fblocks)
@@ -672,7 +672,7 @@ void enqueue_fp64(ed_context* c, const double2* W, int nb, int t_out0, double2* 
   a.nwork = nb * c->f_gt * c->f_nsplit;
   a.order = c->item_order;
   a.t_out0 = t_out0;
-  a.dplan = c->dplan.p;
+  a.dplan = c->dplan64.p;
   a.splits = c->splits.p;
   for (int k = 0; k < 2; ++k) {
     a.ngrp[k] = c->f_ngrp[v][k];
@@ -885,7 +885,8 @@ void build_plan(ed_context* c) {
     c->items_t = items;
   }
 
-  plan_fp64(c, dpl);
+  std::vector<DPlan> dpl64 = dpl;  // the same derivatives, item0 in tile groups
+  plan_fp64(c, dpl64);
 
   // Unit plan of the FP16 stage-1 kernel.  A merged split's coefficient is
   // (-1)^{|nR|} times a positive multiplicity (merged_splits).  With slot n
@@ -937,6 +938,7 @@ void build_plan(ed_context* c) {
     views.push_back([c, &view, at] { view.p = (std::remove_reference_t<decltype(view.p)>)(void*)(c->tabs.p + at); });
   };
   put(c->dplan, dpl);
+  put(c->dplan64, dpl64);
   put(c->splits, sp);
   put(c->pidx, idx);
   put(c->psum, ps);

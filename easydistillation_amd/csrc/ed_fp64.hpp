@@ -82,7 +82,7 @@ struct Args {
   int ngrp[2];       // groups of one derivative: all tiles / tiles te <= tf
   int order;         // 0: CHUNK consecutive items per XCD in turn, 1: round robin
   int nf, ns, nmom, t_out0;
-  const DPlan* dplan;
+  const DPlan* dplan;  // item0: first tile group of the derivative
   const SplitTerm* splits;
   const Group* grp[2];
   const double* xt;  // [Lx + 1][F1]
@@ -409,10 +409,10 @@ __global__ __launch_bounds__(128 * NT_MAX, 1) void contract_kernel(const double2
   const int tb = w / per_t;
   int r = w - tb * per_t;
   int di = 0;
-  while (di + 1 < a.nd && uni(a.dplan[di + 1].grp0) * a.nsplit <= r) ++di;
+  while (di + 1 < a.nd && uni(a.dplan[di + 1].item0) * a.nsplit <= r) ++di;
   DPlan dp = a.dplan[di];
-  dp.first = uni(dp.first), dp.nsplit = uni(dp.nsplit), dp.mirror = uni(dp.mirror), dp.grp0 = uni(dp.grp0);
-  r -= dp.grp0 * a.nsplit;
+  dp.first = uni(dp.first), dp.nsplit = uni(dp.nsplit), dp.mirror = uni(dp.mirror), dp.item0 = uni(dp.item0);
+  r -= dp.item0 * a.nsplit;
   const int ng = dp.mirror ? a.ngrp[1] : a.ngrp[0];
   const int split = r / ng, gi = r - split * ng;
   Group gr = (dp.mirror ? a.grp[1] : a.grp[0])[gi];
@@ -427,7 +427,7 @@ __global__ __launch_bounds__(128 * NT_MAX, 1) void contract_kernel(const double2
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const double2* Wt = W + (size_t)tb * a.g.nW * a.g.V3P * 3 * a.g.NeP;
   const int seg = z0 * a.spp + part;
-  double* Mw = a.M + (((size_t)(tb * a.gt + dp.grp0 + gi) * (a.g.Lz * a.spp) + seg) * a.NT * 2 + wave) * (PAT::NS * 256);
+  double* Mw = a.M + (((size_t)(tb * a.gt + dp.item0 + gi) * (a.g.Lz * a.spp) + seg) * a.NT * 2 + wave) * (PAT::NS * 256);
   const int nq = (6 * dp.nsplit + 3) >> 2;
   auto go = [&](auto n) {
     constexpr int NQ = decltype(n)::value;
@@ -455,9 +455,9 @@ __global__ __launch_bounds__(256) void momenta_kernel(Args a) {
   b /= a.NT;
   const int tb = b / a.gt, gi = b - tb * a.gt;
   int di = 0;
-  while (di + 1 < a.nd && a.dplan[di + 1].grp0 <= gi) ++di;
+  while (di + 1 < a.nd && a.dplan[di + 1].item0 <= gi) ++di;
   const DPlan dp = a.dplan[di];
-  const Group gr = (dp.mirror ? a.grp[1] : a.grp[0])[gi - dp.grp0];
+  const Group gr = (dp.mirror ? a.grp[1] : a.grp[0])[gi - dp.item0];
   if (q >= gr.nT) return;
   const int tile = pick(gr.tile, q), te = pick(gr.rowL, tile & 15), tf = pick(gr.rowR, tile >> 4);
   const int nseg = a.g.Lz * a.spp, wave = uni(threadIdx.x >> 6);

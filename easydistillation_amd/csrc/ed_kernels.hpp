@@ -539,9 +539,8 @@ struct DPlan {
   int first, nsplit;
   int mirror;       // rev(d) = d: only tiles te <= tf run; tile (te, tf) also
                     // writes the transposed tile (tf, te) through the partner rule
-  int item0;        // first work item of this d within a timeslice
+  int item0;        // first work item (FP64: tile group) of this d within a timeslice
   int rot;          // the FP16 stage-1 kernel multiplies its result by i^rot
-  int grp0;         // FP64 contraction: first tile group of this d within a timeslice
 };
 
 // The diagonal tile of a self-partnered derivative computes every (e, f)
